@@ -16,7 +16,7 @@
 //      owns 4 rows, and every score is fmaf over d ascending from 0, then * scale, so the fp32
 //      score is a fixed function of its inputs (reproduced bit for bit by the C oracle).
 //   3. selection, one wave per row: keys in registers; theta = topk-th largest score word of the
-//      64 per-lane maxima (ranked across lanes), past topk 64 the exact topk-th largest score
+//      64 per-lane maxima (ranked across lanes), past topk 56 the exact topk-th largest score
 //      word (wave radix select); only keys at or above it survive;
 //      each survivor's exact rank among survivors is counted from LDS; rank < topk is written.
 //      Column chunk ids are precomputed once per workgroup in LDS.
@@ -132,11 +132,18 @@ __device__ __forceinline__ int row_ub(const MaskDev& m, const RowInfo& r, int NC
 // lanes of the wave must call this; sv is the wave's LDS survivor buffer.
 //   1. every lane loads its keys (candidates lane, lane + 64, ...) into registers once;
 //   2. theta = the topk-th largest high word (score half) of the 64 per-lane maxima, from each
-//      lane's rank among them (readlane compares, no LDS and no scalar round trips);
+//      lane's rank among them; past kLaneMaxTopk the exact topk-th largest high word;
 //   3. survivors = keys whose high word is >= theta (at least topk of them whenever that many
 //      candidates exist, and every key of the top topk), compacted into sv;
 //   4. each survivor's exact rank among the survivors (keys are distinct) -> emit if < topk.
 constexpr int kMaxPer = kSpanCap / kWave;
+// Up to this topk theta comes from the 64 lane maxima, past it from an exact radix select.  The
+// lane maxima cost less, but close to 64 they cut almost nothing: with 16 keys a lane the 56th
+// largest of the 64 maxima leaves about 125 survivors, the 64th (their minimum) about 300, past
+// the survivor buffer, and the row then takes its maxima one at a time.  16380 rows of 1365
+// columns: topk 56 285 us with the maxima and 292 us with the radix select, topk 64 558 and 295 us
+// (4680 tokens over 5920 columns: 119 and 117 us, 283 and 118 us).
+constexpr int kLaneMaxTopk = 56;
 
 // Wave-wide max of an unsigned value (DPP row shifts and row broadcasts; every lane gets it).
 template <int CTRL, int ROW_MASK>
@@ -155,11 +162,10 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
   return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), kWave - 1));
 }
 
-// The topk-th largest of the 64 lane values v (0 if topk > 64): every lane counts the values
+// The topk-th largest of the 64 lane values v: every lane counts the values
 // >= its own (64 LDS broadcast values in the wave-private scratch), and the answer is the
 // largest value whose count reaches topk.  scratch: 64 words of wave-private LDS.
 __device__ __forceinline__ uint32_t lane_max_threshold(uint32_t v, int topk, uint32_t* scratch) {
-  if (topk > kWave) return 0u;
   const int lane = lane_id();
   scratch[lane] = v;
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -178,7 +184,7 @@ __device__ __forceinline__ uint32_t lane_max_threshold(uint32_t v, int topk, uin
   return theta;
 }
 
-// For 64 < topk <= 128: the exact topk-th largest high word among the wave's candidates, by a
+// Past kLaneMaxTopk: the exact topk-th largest high word among the wave's candidates, by a
 // radix select over the 32-bit high words (4 passes of 8 bits, each a 256-bin histogram in the
 // wave's LDS scratch and a scan of the bins from the top), so that about topk keys survive.  1
 // when fewer than topk candidates exist (every candidate passes: candidates have a high word
@@ -261,9 +267,9 @@ __device__ __forceinline__ void wave_select_impl(int n, int topk, KeyF key, Emit
     const uint32_t h = static_cast<uint32_t>(kv[j] >> 32);
     lmax = h > lmax ? h : lmax;
   }
-  // theta: the topk-th largest lane maximum (0 if fewer than topk lanes hold candidates); past
-  // 64, the exact topk-th largest high word
-  const uint32_t theta = topk <= kWave
+  // theta: the topk-th largest lane maximum (0 if fewer than topk lanes hold candidates), or the
+  // exact topk-th largest high word
+  const uint32_t theta = topk <= kLaneMaxTopk
       ? lane_max_threshold(lmax, topk, reinterpret_cast<uint32_t*>(sv))
       : wave_radix_threshold(
             PER, topk,
@@ -376,7 +382,7 @@ __device__ __forceinline__ void wave_select_stream(int n, int topk, KeyF key, Em
       lmax = h > lmax ? h : lmax;
     }
   }
-  const uint32_t theta = topk <= kWave
+  const uint32_t theta = topk <= kLaneMaxTopk
       ? lane_max_threshold(lmax, topk, reinterpret_cast<uint32_t*>(sv))
       : wave_radix_threshold(
             per, topk,

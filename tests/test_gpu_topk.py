@@ -102,6 +102,19 @@ def test_topk_from_scores_bitexact(mask, topk, NC):
     np.testing.assert_array_equal(got, want)
 
 
+@pytest.mark.parametrize("topk", [55, 56, 57, 63, 64])
+@pytest.mark.parametrize("NC", [64, 257, 1024, 1025])
+@pytest.mark.parametrize("ties", [False, True])
+def test_topk_from_scores_threshold_edges_bitexact(topk, NC, ties):
+    """Around the topk where the survivor threshold changes from the lane maxima to the radix
+    select, with 1, 5 and 16 keys a lane and one column past a span."""
+    from omnimem_amd.index_topk import topk_from_scores
+    mk = MASKS["noncausal"]
+    s = _scores_case(topk * 7 + NC + ties, 1, 9, 2, NC, ties=ties)
+    got = topk_from_scores(torch.from_numpy(s).to(DEV), topk, 64, 64, 64, False).cpu().numpy()
+    np.testing.assert_array_equal(got, O.topk_select(s, topk, O.Mask(**mk)))
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("topk", [96, 128])
 def test_parallel_nsa_topk_fused_large_topk_bitexact(dtype, topk):
