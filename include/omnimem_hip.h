@@ -2,8 +2,8 @@
  * omnimem_hip.h -- C ABI of the MI355X (gfx950) native-sparse-attention selection path.
  *
  * Every entry point takes plain device pointers, element strides and sizes, runs on the HIP
- * stream it is given (passed as void*, a hipStream_t), never synchronises, and returns an
- * OMM_* status.  On failure omm_last_error() returns a thread-local message.  No entry point
+ * stream it is given (passed as void*, a hipStream_t), never synchronises (but for
+ * omm_ids_check_end, which waits for one check), and returns an OMM_* status.  On failure omm_last_error() returns a thread-local message.  No entry point
  * allocates device memory: scratch is passed in by the caller (see the *_workspace_bytes
  * queries), so a caller's caching allocator owns every byte.
  *
@@ -51,6 +51,8 @@
  *   omm_copy_units_async    <- flush_offload's D2H copies (models/cache.py:1086-1117) on the
  *                              copy engines
  *   omm_host_alloc / _free  <- MMCache's pinned offload buffers (models/cache.py:970-1016)
+ *   omm_ids_check_begin / _end <- the facade's block-id range check
+ *                              (nsa/ops/selection/__init__.py:36-42)
  *   omm_topk_fused_noalloc, omm_topk_fused_debug: no reference counterpart (callers that cannot
  *                              allocate; a test hook that also returns the scores)
  */
@@ -171,6 +173,15 @@ int omm_abi_version(void); /* 4 */
  * (models/cache.py:970-1016) and the pinned tensors of its eviction path (cache.py:853,906). */
 int omm_host_alloc(size_t bytes, void** host, void** dev);
 int omm_host_free(void* host);
+
+/* Range check of selection block ids: begin enqueues one kernel that looks for an id >=
+ * num_blocks (negative ids mean "no block" and pass) and returns a ticket, NULL when no id can be
+ * out of range; end waits for that kernel, not for work enqueued after it, sets *bad to 1 if it
+ * found one and releases the ticket (every ticket is ended once).  The selection kernels skip
+ * out-of-range ids, so a caller enqueues them between the two and discards their result on an
+ * error.  Not for a stream under capture.  ids: int32, on the current device. */
+int omm_ids_check_begin(const omm_view4* ids, int64_t num_blocks, void* stream, void** ticket);
+int omm_ids_check_end(void* ticket, int32_t* bad);
 
 /* ---- block compression / query pooling (a1, a2) -------------------------------------- */
 /* out[b, j, h, :] = mean over tokens t in [j*group, min((j+1)*group, T)) of x[b, t, h, :].

@@ -68,6 +68,8 @@ PROTOTYPES = {
     "omm_abi_version": (_i32, []),
     "omm_host_alloc": (_i32, [_sz, ctypes.POINTER(_vp), ctypes.POINTER(_vp)]),
     "omm_host_free": (_i32, [_vp]),
+    "omm_ids_check_begin": (_i32, [_V, _i64, _vp, ctypes.POINTER(_vp)]),
+    "omm_ids_check_end": (_i32, [_vp, ctypes.POINTER(_i32)]),
     "omm_block_pool": (_i32, [_V, _V, _i32, _i32, _vp]),
     "omm_topk_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64, _i32]),
     "omm_topk": (_i32, [_V, _V, _i32, _i32, _f32, _M, _vp, _vp, _sz, _vp]),

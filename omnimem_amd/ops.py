@@ -90,9 +90,39 @@ def check_block_ids_now(block_indices, num_blocks):
     synchronisation, ValueError for a valid id >= num_blocks."""
     valid_mask = block_indices >= 0
     if valid_mask.any() and torch.any(block_indices[valid_mask] >= num_blocks):
-        raise ValueError(
-            f"top_idx out of range: expected in [-1, {num_blocks - 1}] "
-            f"but got [{block_indices.min()}, {block_indices.max()}]")
+        raise _block_ids_error(block_indices, num_blocks)
+
+
+def begin_block_ids_check(block_indices, num_blocks):
+    """``check_block_ids_now`` in two halves: enqueues the check and returns the function that
+    waits for it and raises, to be called once the work behind it is enqueued.  The wait then
+    overlaps that work.  Anything but plain int32 ids on the current device outside of a capture
+    or a dispatch mode is checked here and now."""
+    if not (type(block_indices) is torch.Tensor and block_indices.is_cuda
+            and block_indices.dtype == torch.int32 and block_indices.dim() == 4
+            and block_indices.device.index == torch.cuda.current_device()
+            and not torch._C._functorch.is_functorch_wrapped_tensor(block_indices)
+            and torch._C._len_torch_dispatch_stack() == 0
+            and not torch.cuda.is_current_stream_capturing()):
+        check_block_ids_now(block_indices, num_blocks)
+        return lambda: None
+    from . import _lib
+    ticket = _lib.ctypes.c_void_p()
+    _lib.call("omm_ids_check_begin", _lib.view4(block_indices), int(num_blocks),
+              _lib.stream_of(block_indices), _lib.ctypes.byref(ticket))
+
+    def finish():
+        bad = _lib.ctypes.c_int32()
+        _lib.call("omm_ids_check_end", ticket, _lib.ctypes.byref(bad))
+        if bad.value:
+            raise _block_ids_error(block_indices, num_blocks)
+    return finish
+
+
+def _block_ids_error(block_indices, num_blocks):
+    return ValueError(
+        f"top_idx out of range: expected in [-1, {num_blocks - 1}] "
+        f"but got [{block_indices.min()}, {block_indices.max()}]")
 
 
 def _check_block_ids_impl(sink, block_indices, num_blocks):

@@ -25,8 +25,9 @@ def _debug_checks_enabled() -> bool:
     return os.environ.get("OMNIMEM_NSA_DEBUG", "0") not in ("", "0", "false", "False")
 
 
-def _validate_common(q, k, v, block_indices, block_size, chunk_size, group_size, causal):
-    """Argument checks of the reference facade (nsa/ops/selection/__init__.py:16-44)."""
+def _validate_shapes(q, k, v, block_indices, block_size, chunk_size, group_size):
+    """Argument checks of the reference facade but for the id range
+    (nsa/ops/selection/__init__.py:16-35); returns the number of blocks."""
     B, M, H, D = q.shape
     N = k.shape[1]
     G = group_size
@@ -40,7 +41,12 @@ def _validate_common(q, k, v, block_indices, block_size, chunk_size, group_size,
         raise ValueError(f"chunk_size must be > 0, got {chunk_size}")
     if block_indices.shape[-1] == 0:
         raise ValueError("top_idx last dim T must be > 0")
-    num_blocks = math.ceil(N / block_size)
+    return math.ceil(N / block_size)
+
+
+def _validate_common(q, k, v, block_indices, block_size, chunk_size, group_size, causal):
+    """Argument checks of the reference facade (nsa/ops/selection/__init__.py:16-44)."""
+    num_blocks = _validate_shapes(q, k, v, block_indices, block_size, chunk_size, group_size)
     # One host sync per call, as in the reference; the op-level sel_fwd() skips it.  A traced
     # graph cannot branch on tensor values, so there the same check runs as an op of the graph
     # and raises the same ValueError when the graph runs.
@@ -235,9 +241,25 @@ def selection_attention(
     if bwd_method not in ('auto', 'mask', 'inverted'):
         raise ValueError(f"Unknown bwd_method '{bwd_method}', expected 'auto', 'inverted' or 'mask'")
     get_backend()
-    _validate_common(q, k, v, block_indices, block_size, chunk_size, group_size, causal)
-    if not torch.compiler.is_compiling() and _debug_checks_enabled():
-        _debug_check_unique(block_indices)
+    args = (q, k, v, block_indices, block_size, chunk_size, scale, causal, return_lse, allow_tf32,
+            bwd_method, group_size)
+    if torch.compiler.is_compiling():
+        _validate_common(q, k, v, block_indices, block_size, chunk_size, group_size, causal)
+        return _selection_attention(*args)
+    # the id check is enqueued first and waited for once the attention is enqueued behind it
+    finish = ops.begin_block_ids_check(
+        block_indices, _validate_shapes(q, k, v, block_indices, block_size, chunk_size, group_size))
+    try:
+        if _debug_checks_enabled():
+            _debug_check_unique(block_indices)
+        return _selection_attention(*args)
+    finally:
+        finish()
+
+
+def _selection_attention(q, k, v, block_indices, block_size, chunk_size, scale, causal, return_lse,
+                         allow_tf32, bwd_method, group_size):
+    """``selection_attention`` after its checks."""
     if block_indices.dtype != torch.int32:
         block_indices = block_indices.to(torch.int32)
     sc = scale if scale is not None else q.shape[-1] ** -0.5

@@ -401,3 +401,43 @@ def test_sel_fwd_gated_rejects_overlap_and_bad_inputs():
     with pytest.raises(NSABackendError, match="gates"):
         call(g_=torch.rand((1, M, H, 2), device=DEV).to(dt))
     assert torch.isfinite(call().float()).all()
+
+
+@pytest.mark.parametrize("form", ["flat", "offset", "expanded", "transposed", "int64"])
+@pytest.mark.parametrize("at", ["first", "last", "none"])
+def test_id_range_check_every_layout(form, at):
+    """The facade refuses an id of ceil(N / block) wherever it sits and whatever the layout of the
+    ids (flat 16-byte reads with a remainder, a misaligned start, a view with strides), with
+    gradients too, passes -1 and the largest id, and works again after an error."""
+    from omnimem_amd.selection import selection_attention
+    g = torch.Generator().manual_seed(3)
+    M, N, H, T, G = 192, 200, 3, 5, 64  # 45 ids, blocks 0 .. 3 (the last of 8 tokens)
+    q, k, v = (torch.randn((1, n, H, 64), generator=g).bfloat16().cuda() for n in (M, N, N))
+    ids = torch.randint(-1, 4, (1, M // G, H, T), generator=g, dtype=torch.int32)
+    if form == "expanded":
+        ids = ids[:, :1].clone()
+    if at != "none":
+        ids[(0,) * 4 if at == "first" else (-1,) * 4] = 4
+    if form == "int64":
+        ids = ids.long()
+        if at != "none":
+            ids[ids == 4] = 2 ** 32 + 1  # in range once truncated to 32 bits
+    ids = ids.cuda()
+    if form == "offset":
+        ids = torch.cat([ids.new_zeros(1), ids.flatten()])[1:].view(ids.shape)
+    elif form == "expanded":
+        ids = ids.expand(1, M // G, H, T)
+    elif form == "transposed":
+        ids = ids.permute(0, 3, 2, 1).contiguous().permute(0, 3, 2, 1)
+    for grad in (False, True):
+        qq = q.clone().requires_grad_(grad)
+        if at == "none":
+            out = selection_attention(qq, k, v, ids, T, 64, group_size=G)
+            assert torch.isfinite(out.float()).all()
+            continue
+        with pytest.raises(ValueError, match="top_idx out of range: expected in .-1, 3."):
+            selection_attention(qq, k, v, ids, T, 64, group_size=G)
+    ok = torch.where(ids >= 4, 3, ids)
+    a = selection_attention(q, k, v, ok, T, 64, group_size=G)
+    b = selection_attention(q, k, v, ok.int().contiguous(), T, 64, group_size=G)
+    assert torch.equal(a, b)
