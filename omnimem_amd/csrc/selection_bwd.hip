@@ -432,23 +432,27 @@ __global__ __launch_bounds__(kIdxThreads) void sel_bwd_index_kernel(
 }
 
 // ---- dK / dV ----------------------------------------------------------------------------------
-// Workgroup = 4 waves over one 64-key tile: wave w owns keys 16 w .. 16 w + 15 (one MFMA column
-// block) for every query of every item.  Its K / V operands and fp32 dK / dV sums take ~100
-// registers, so two waves share each SIMD (the workgroup's 66 KiB of LDS allows two workgroups
-// per CU) and one wave's LDS and memory waits are covered by the other's work.  The item's lse arrives
-// already as -lse log2 e (written by the dQ kernel), and the softmax scale of dK is applied once
-// to the sums.
-constexpr int kKvThreads = 256;
+// Workgroup = NW waves over one tile of 16 NW keys: wave w owns keys 16 w .. 16 w + 15 (one MFMA
+// column block) for every query of every item.  Its K / V operands and fp32 dK / dV sums take ~100
+// registers, so two waves share each SIMD (LDS: 66 KiB for 4 waves, 33 KiB for 2) and one wave's
+// LDS and memory waits are covered by the other's work.  The item's lse arrives already as
+// -lse log2 e (written by the dQ kernel), and the softmax scale of dK is applied once to the sums.
+//
+// The kernel is bound by its LDS reads (every wave reads each Q / dO row twice, as rows and
+// transposed: 16 KiB per 16 queries and 16 keys, 128 cycles of the CU's LDS against 256 of one
+// SIMD's MFMA), so rows without a query and columns without a key cost as much as real ones.  Hence
+// SUB: a tile of 16 NW query rows holds 16 NW / SUB bucket items of up to SUB queries (SUB = 16 for
+// query groups of at most 16, else 32), from as many groups.  And NW = 2 for blocks of at most 32
+// keys, which would leave two of four waves without one.
 
-// One dword per lane: lane L's float at base + 4 L (lanes at or past nvalid read 0) into LDS
-// dst + 4 L, issued like dma_part (inline asm, ordered by the kernel's own waits).
+// One dword per lane: lane L's float at byte off of base (off < 0: 0) into LDS dst + 4 L, issued
+// like dma_part (inline asm, ordered by the kernel's own waits).
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
-__device__ __forceinline__ void dma_f32x64(const float* base, int nvalid, float* dst) {
-  const i32x4 r = buffer_desc(base, 4 * nvalid);
+__device__ __forceinline__ void dma_f32x64(const float* base, int off, float* dst) {
+  const i32x4 r = buffer_desc(base, 0x7fffffff);
   const uint32_t m0 = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(
       static_cast<int>(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(dst)))));
-  const int off = 4 * lane_id();
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds"
                :
                : "s"(m0), "v"(off), "s"(r)
@@ -457,7 +461,7 @@ __device__ __forceinline__ void dma_f32x64(const float* base, int nvalid, float*
 #pragma clang diagnostic pop
 
 // ---- dK / dV targets --------------------------------------------------------------------------
-// One key tile (up to 64 tokens) of one (b, h, block): element pointers of its first K / V row and
+// One key tile (up to KT tokens) of one (b, h, block): element pointers of its first K / V row and
 // first dK / dV row, element strides, its row count and the token id of its first row (used by the
 // chunk-causal mask only).
 template <typename KT, typename GT>
@@ -479,9 +483,10 @@ struct DenseGrad {
   View4<const QT> k, v;
   View4<QT> dk, dv;
   int N, bs;
+  template <int KT>
   __device__ __forceinline__ bool tile(int b, int h, int bid, int kt, KvTile<QT, QT>& r) const {
-    const int t0 = bid * bs + 64 * kt;
-    const int nk = min(min(bs - 64 * kt, 64), N - t0);
+    const int t0 = bid * bs + KT * kt;
+    const int nk = min(min(bs - KT * kt, KT), N - t0);
     if (nk <= 0) return false;
     r = KvTile<QT, QT>{k.at(b, t0, h), v.at(b, t0, h), dk.at(b, t0, h), dv.at(b, t0, h),
                        k.s1, k.s3, v.s1, v.s3, dk.s1, dk.s3, dv.s1, dv.s3, nk, t0};
@@ -509,6 +514,7 @@ struct PtrGrad {
   int64_t batch_kv, batch_dkv, chunk_kv, chunk_dkv;  // bytes
   int64_t s_bn, s_bd, s_dbn, s_dbd;                  // element strides
   int bpc, bs;
+  template <int KT>
   __device__ __forceinline__ bool tile(int b, int h, int bid, int kt, KvTile<bf16_t, float>& r) const {
     if (n_blocks != nullptr && bid >= n_blocks[h]) return false;
     const int64_t idx = bpc > 0 ? bid / bpc : bid;
@@ -517,10 +523,10 @@ struct PtrGrad {
     const int64_t o = h * bsh + idx * bsc;
     const int64_t bk = base_k[o], bv = base_v[o], bdk = base_dk[o], bdv = base_dv[o];
     if (bk == 0 || bv == 0 || bdk == 0 || bdv == 0) return false;
-    const int nk = min(bs - 64 * kt, 64);
+    const int nk = min(bs - KT * kt, KT);
     if (nk <= 0) return false;
     const int64_t okv = b * batch_kv + loc * chunk_kv, od = b * batch_dkv + loc * chunk_dkv;
-    const int64_t row0 = 64 * static_cast<int64_t>(kt);
+    const int64_t row0 = KT * static_cast<int64_t>(kt);
     r.k = reinterpret_cast<const bf16_t*>(static_cast<uintptr_t>(bk + okv)) + row0 * s_bn;
     r.v = reinterpret_cast<const bf16_t*>(static_cast<uintptr_t>(bv + okv)) + row0 * s_bn;
     r.dk = reinterpret_cast<float*>(static_cast<uintptr_t>(bdk + od)) + row0 * s_dbn;
@@ -572,22 +578,25 @@ __device__ __forceinline__ void store_row8(float* p, int64_t sd, const float4& x
   for (int i = 0; i < 8; ++i) p[i * sd] = x[i];
 }
 
-template <typename QT, int D, typename KG>
-__global__ __launch_bounds__(kKvThreads, 2) void sel_bwd_dkv_kernel(
+template <typename QT, int D, typename KG, int NW, int SUB>
+__global__ __launch_bounds__(NW * kWave, 2) void sel_bwd_dkv_kernel(
     View4<const QT> q, View4<const QT> dout, KG kg, const float* __restrict__ nl2,
     const float* __restrict__ delta, const int32_t* __restrict__ offsets,
     const int32_t* __restrict__ groups, int M, int H, int G, int MG, int T, int NS, int nkt,
-    int chunk, bool causal, float scale, int nsub) {
+    int chunk, bool causal, float scale, int nparts) {
   using DG = DmaGeom<D>;
   constexpr int ROWB = DG::ROWB, CPR = DG::CPR, RPI = DG::RPI;
   constexpr int SD = DG::SD, ND = DG::ND;
-  constexpr int QB = 64 * ROWB;           // bytes of one 64-row Q or dO tile
-  constexpr int NPC = QB / 4096;          // 4 KiB copy pieces per tile (4 copy instructions)
-  constexpr int PPW = 2 * NPC / 4;        // pieces per wave (Q and dO pieces of both tiles)
+  constexpr int KT = 16 * NW;             // keys per workgroup
+  constexpr int QR = 16 * NW;             // query rows per tile
+  constexpr int SPT = QR / SUB;           // bucket items per tile
+  constexpr int QB = QR * ROWB;           // bytes of one Q or dO tile
+  constexpr int NI = 16 / RPI;            // copy instructions per 16 rows
+  static_assert(2 * (QR / 16) == 2 * NW, "two 16-row copies per wave: one of Q, one of dO");
   // [Q buffer 0, Q buffer 1, dO buffer 0, dO buffer 1][QB] then [buffer][lse, delta][64]
   __shared__ __align__(16) char smem[4 * QB + 2 * 2 * 64 * 4];
 
-  const int tid = static_cast<int>(threadIdx.x), lane = lane_id(), w = tid / kWave;
+  const int tid = static_cast<int>(threadIdx.x), lane = lane_id(), w = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int l16 = lane & 15, j4 = lane >> 4;
   // Work order.  A key block's work is the number of query groups that selected it; under a
   // causal chunk mask the early blocks are picked by many more groups than the late ones.  Units
@@ -614,7 +623,7 @@ __global__ __launch_bounds__(kKvThreads, 2) void sel_bwd_dkv_kernel(
   const int b = u / H;
 
   KvTile<typename KG::KT, typename KG::GT> tl;
-  if (!kg.tile(b, h, bid, kt, tl)) return;
+  if (!kg.template tile<KT>(b, h, bid, kt, tl)) return;
   const int t0 = tl.t0, nk = tl.nk;  // first token and tokens of the tile
 
   // K^T and V^T operands of this wave's key 16 w + l16, dims 32 s + 8 j4 ..
@@ -646,14 +655,16 @@ __global__ __launch_bounds__(kKvThreads, 2) void sel_bwd_dkv_kernel(
   const int tx = DG::swz_v(tr) >> 1;
   auto roff = [&](int s) { return rbase + ((rx ^ (4 * s)) << 4); };
   auto troff = [&](int i) { return tbase + ((i ^ tx) << 5); };
-  // copy pieces of this wave: piece p = w + 4 pp of [Q pieces 0 .. NPC-1, dO pieces 0 .. NPC-1];
-  // instruction jj of piece pc copies rows (4 pc + jj) RPI + lane / CPR, whose row modulo 8
-  // (and so swizzle) does not depend on pc
+  // this wave copies rows 16 w .. 16 w + 15 of the Q and of the dO tile; instruction jj of a copy
+  // takes rows jj RPI + lane / CPR of them, whose row modulo 8 (and so swizzle) is that of the tile
   const int rsq = static_cast<int>(q.s1) * 2, rsd = static_cast<int>(dout.s1) * 2;
-  const int crow = lane / CPR;
-  int csw[4];
+  int qo[NI], dof[NI];
 #pragma unroll
-  for (int jj = 0; jj < 4; ++jj) csw[jj] = ((lane % CPR) ^ DG::swz_v(jj * RPI + crow)) << 4;
+  for (int jj = 0; jj < NI; ++jj) {
+    const int row = jj * RPI + lane / CPR, c = ((lane % CPR) ^ DG::swz_v(row)) << 4;
+    qo[jj] = row * rsq + c;
+    dof[jj] = row * rsd + c;
+  }
 
   // dK / scale and dV of keys 16 w + 4 j4 + r, dims 16 i + l16
   f32x4 acc_dk[ND], acc_dv[ND];
@@ -663,13 +674,15 @@ __global__ __launch_bounds__(kKvThreads, 2) void sel_bwd_dkv_kernel(
   const int64_t orow = (static_cast<int64_t>(b) * H + h) * (NS + 1);
   const int e0 = offsets[orow + bid], e1 = offsets[orow + bid + 1];
   const int32_t* grp = groups + (static_cast<int64_t>(b) * H + h) * (static_cast<int64_t>(MG) * T);
-  const int nitems = (e1 - e0) * nsub;
+  const int nitems = (e1 - e0) * nparts;
   const int64_t lrow = (static_cast<int64_t>(b) * H + h) * M;
 
-  // item i = (bucket entry i / nsub, 64-query part i % nsub): its first query, queries and
-  // visible keys of this tile; find() returns the next item with work at or after i
-  struct Item {
-    int i, q0, nq, nv;
+  // item i = (bucket entry i / nparts, SUB-query part i % nparts): its first query, queries and
+  // visible keys of this key tile.  A tile holds the next SPT items with work (an item that is
+  // missing at the end has no queries and no keys); next is the first item after them.
+  struct Tile {
+    int q0[SPT], nq[SPT], nv[SPT];
+    int next;
   };
   // bucket entries held in a VGPR, 64 at a time (lane j: entry gwin + j), read with readlane
   int gwin = -64, gv = 0;
@@ -680,57 +693,76 @@ __global__ __launch_bounds__(kKvThreads, 2) void sel_bwd_dkv_kernel(
     }
     return __builtin_amdgcn_readlane(gv, e & 63);
   };
-  auto find = [&](int i) -> Item {
-    for (; i < nitems; ++i) {
-      const int e = i / nsub, part = i - (i / nsub) * nsub;
-      const int g = group_of(e);
-      const int q0 = g * G + 64 * part;
-      const int nq = min(min(g * G + G, M) - q0, 64);
-      int nv = nk;
-      if (causal) {
-        const int64_t lim = static_cast<int64_t>((g * G) / chunk + 1) * chunk - t0;
-        nv = lim < nv ? static_cast<int>(lim > 0 ? lim : 0) : nv;
+  auto find = [&](int i) -> Tile {
+    Tile t;
+#pragma unroll
+    for (int c = 0; c < SPT; ++c) {
+      t.q0[c] = t.nq[c] = t.nv[c] = 0;
+      for (; i < nitems; ++i) {
+        const int e = nparts == 1 ? i : i / nparts, part = i - e * nparts;
+        const int g = group_of(e);
+        const int q0 = g * G + SUB * part;
+        const int nq = min(min(g * G + G, M) - q0, SUB);
+        int nv = nk;
+        if (causal) {
+          const int64_t lim = static_cast<int64_t>((g * G) / chunk + 1) * chunk - t0;
+          nv = lim < nv ? static_cast<int>(lim > 0 ? lim : 0) : nv;
+        }
+        if (nq > 0 && nv > 0) {
+          t.q0[c] = q0;
+          t.nq[c] = nq;
+          t.nv[c] = nv;
+          ++i;
+          break;
+        }
       }
-      if (nq > 0 && nv > 0) return Item{i, q0, nq, nv};
     }
-    return Item{nitems, 0, 0, 0};
+    t.next = i;
+    return t;
   };
-  auto issue = [&](const Item& it, int buf) {
-    const char* qbase = reinterpret_cast<const char*>(q.at(b, it.q0, h, 0));
-    const char* dbase = reinterpret_cast<const char*>(dout.at(b, it.q0, h, 0));
+  // Copies of a tile into buffers buf: this wave's 16 rows of Q and of dO, and by waves 0 and 1
+  // every row's -lse log2 e and delta (rows past an item's queries read as 0).
+  auto issue = [&](const Tile& t, int buf) {
+    int q0 = 0, nr = 0;  // of this wave's 16 rows (wave-uniform)
 #pragma unroll
-    for (int pp = 0; pp < PPW; ++pp) {
-      const int piece = w + 4 * pp, pc = piece % NPC;
-      const bool isq = piece < NPC;
-      const int rs = isq ? rsq : rsd;
-      int off[4];
+    for (int c = 0; c < SPT; ++c)
+      if (16 * w / SUB == c) {
+        q0 = t.q0[c] + (16 * w) % SUB;
+        nr = min(max(t.nq[c] - (16 * w) % SUB, 0), 16);
+      }
+    q0 = nr > 0 ? q0 : 0;
+    dma_part<NI>(q.at(b, q0, h, 0), rsq, nr, smem + buf * QB + 16 * w * ROWB, 0, qo);
+    dma_part<NI>(dout.at(b, q0, h, 0), rsd, nr, smem + (2 + buf) * QB + 16 * w * ROWB, 0, dof);
+    if (w < 2) {
+      // offsets from the tile's first query: a bucket's groups ascend, and M < 2^29
+      int off = -1;
 #pragma unroll
-      for (int jj = 0; jj < 4; ++jj) off[jj] = ((4 * pc + jj) * RPI + crow) * rs + csw[jj];
-      dma_part(isq ? qbase : dbase, rs, it.nq, smem + (isq ? buf : 2 + buf) * QB, pc, off);
-    }
-    if (w < 2)
-      dma_f32x64((w == 0 ? nl2 : delta) + lrow + it.q0, it.nq,
+      for (int c = 0; c < SPT; ++c) {
+        const int r = lane - SUB * c;
+        if (r >= 0 && r < t.nq[c]) off = 4 * (t.q0[c] - t.q0[0] + r);
+      }
+      dma_f32x64((w == 0 ? nl2 : delta) + lrow + t.q0[0], off,
                  reinterpret_cast<float*>(smem + 4 * QB) + (buf * 2 + w) * 64);
+    }
   };
 
-  Item cur = find(0);
-  if (cur.i < nitems) issue(cur, 0);
+  Tile cur = find(0);
+  if (cur.nq[0] > 0) issue(cur, 0);
   __builtin_amdgcn_s_waitcnt(0);
 
   int BI = 0;
-  while (cur.i < nitems) {
+  while (cur.nq[0] > 0) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    const Item nx = find(cur.i + 1);
-    if (nx.i < nitems) issue(nx, BI ^ 1);
+    const Tile nx = find(cur.next);
+    if (nx.nq[0] > 0) issue(nx, BI ^ 1);
     const char* Qt = smem + BI * QB;
     const char* Dt = smem + (2 + BI) * QB;
     const float* Ls = reinterpret_cast<const float*>(smem + 4 * QB) + BI * 128;
     const float* Ds = Ls + 64;
-    const bool kv = 16 * w + l16 < cur.nv;
 
 #pragma unroll
-    for (int hq = 0; hq < 2; ++hq) {  // queries 32 hq .. 32 hq + 31
+    for (int hq = 0; hq < QR / 32; ++hq) {  // queries 32 hq .. 32 hq + 31
       // S = Q K^T and dP = dO V^T: lane holds queries 32 hq + 16 x + 4 j4 + r of key 16 w + l16
       f32x4 s4[2], p4[2];
 #pragma unroll
@@ -750,6 +782,7 @@ __global__ __launch_bounds__(kKvThreads, 2) void sel_bwd_dkv_kernel(
       for (int x = 0; x < 2; ++x) {
         const float4 L4 = *reinterpret_cast<const float4*>(Ls + 32 * hq + 16 * x + 4 * j4);
         const float4 D4 = *reinterpret_cast<const float4*>(Ds + 32 * hq + 16 * x + 4 * j4);
+        const bool kv = 16 * w + l16 < cur.nv[(32 * hq + 16 * x) / SUB];
         const float Lr[4] = {L4.x, L4.y, L4.z, L4.w}, Dr[4] = {D4.x, D4.y, D4.z, D4.w};
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -784,11 +817,11 @@ __global__ __launch_bounds__(kKvThreads, 2) void sel_bwd_dkv_kernel(
     BI ^= 1;
   }
 
-  // stage the fp32 key rows ([dK, dV][64 keys][D], 64 KiB: the Q / dO buffers) so that the
+  // stage the fp32 key rows ([dK, dV][KT keys][D]: the Q / dO buffers) so that the
   // whole workgroup converts 8 values at a time (packed conversions) and stores 16 bytes per
   // lane; no copy is in flight here (the last item issued none)
   float* stage = reinterpret_cast<float*>(smem);
-  static_assert(4 * QB >= 2 * 64 * D * 4, "staging area");
+  static_assert(4 * QB >= 2 * KT * D * 4, "staging area");
   __syncthreads();
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
@@ -796,18 +829,18 @@ __global__ __launch_bounds__(kKvThreads, 2) void sel_bwd_dkv_kernel(
 #pragma unroll
     for (int i = 0; i < ND; ++i) {
       stage[key * D + 16 * i + l16] = acc_dk[i][r] * scale;
-      stage[(64 + key) * D + 16 * i + l16] = acc_dv[i][r];
+      stage[(KT + key) * D + 16 * i + l16] = acc_dv[i][r];
     }
   }
   __syncthreads();
   constexpr int CH = D / 8;  // 8-element chunks per row
-  for (int c = tid; c < 2 * 64 * CH; c += kKvThreads) {
+  for (int c = tid; c < 2 * KT * CH; c += NW * kWave) {
     const int row = c / CH, ch = c - (c / CH) * CH;
-    const int key = row & 63;
+    const int key = row & (KT - 1);
     if (key >= nk) continue;
     const float4 x0 = *reinterpret_cast<const float4*>(stage + row * D + 8 * ch);
     const float4 x1 = *reinterpret_cast<const float4*>(stage + row * D + 8 * ch + 4);
-    if (row < 64)
+    if (row < KT)
       store_row8(tl.dk + key * tl.dk_sn + 8 * ch * tl.dk_sd, tl.dk_sd, x0, x1);
     else
       store_row8(tl.dv + key * tl.dv_sn + 8 * ch * tl.dv_sd, tl.dv_sd, x0, x1);
@@ -946,7 +979,7 @@ __global__ __launch_bounds__(256) void sel_bwd_dkv_valu_kernel(
   using KT = typename KG::KT;
   using GT = typename KG::GT;
   KvTile<KT, GT> tl;
-  if (!kg.tile(b, h, bid, kt, tl)) return;
+  if (!kg.template tile<64>(b, h, bid, kt, tl)) return;
   const int t0 = tl.t0, nk = tl.nk;
   const int key = tid >> 2, part = tid & 3, d0 = part * DQ;
   const bool k_ok = key < nk;
@@ -1049,6 +1082,36 @@ inline bool rows16(const omm_view4& x, int64_t D) {
          x.stride[2] % 8 == 0 && x.stride[1] >= D && 2 * x.stride[1] * 64 < (int64_t{1} << 31);
 }
 
+// The dK / dV kernel for a call's block and group size (DM = 64 or 128): 2 waves for blocks of at
+// most 32 keys, 16- or 32-row items for groups of at most 16 or 32 queries.  32760 tokens, 12
+// heads, top-16, blocks of 30 and groups of 15: 1873 us with 4 waves and 64-row items, 432 us now;
+// blocks and groups of 64 keep those (555-600 us; 32-row items in pairs took 8% longer there).
+template <typename QT, int DM, typename KG>
+int launch_dkv(const omm_view4& q, const omm_view4& dout, const KG& kg, const float* nl2,
+               const float* delta, const int32_t* offsets, const int32_t* groups, int M, int H,
+               int G, int MG, int T, int NS, int bs, int chunk, bool causal, float scale,
+               hipStream_t s) {
+  const int64_t bh = q.size[0] * H;
+  auto run = [&](auto nw, auto sub) {
+    constexpr int NW = decltype(nw)::value, SUB = decltype(sub)::value;
+    const int nkt = (bs + 16 * NW - 1) / (16 * NW);
+    sel_bwd_dkv_kernel<QT, DM, KG, NW, SUB>
+        <<<static_cast<unsigned>(bh * NS * nkt), NW * kWave, 0, s>>>(
+            make_view<const QT>(q), make_view<const QT>(dout), kg, nl2, delta, offsets, groups, M,
+            H, G, MG, T, NS, nkt, chunk, causal, scale, (G + SUB - 1) / SUB);
+  };
+  using std::integral_constant;
+  if (bs <= 32) {
+    if (G <= 16) run(integral_constant<int, 2>{}, integral_constant<int, 16>{});
+    else run(integral_constant<int, 2>{}, integral_constant<int, 32>{});
+  } else {
+    if (G <= 16) run(integral_constant<int, 4>{}, integral_constant<int, 16>{});
+    else if (G <= 32) run(integral_constant<int, 4>{}, integral_constant<int, 32>{});
+    else run(integral_constant<int, 4>{}, integral_constant<int, 64>{});
+  }
+  return check_launch("selection backward (dk/dv)");
+}
+
 struct BwdArgs {
   const omm_view4 *q, *k, *v, *ids, *out, *dout, *dq, *dk, *dv;
   const float* lse;
@@ -1113,9 +1176,8 @@ int sel_bwd_launch(const BwdArgs& a, char* ws, const BwdWs& L, hipStream_t s) {
   const DenseGrad<QT> kg{make_view<const QT>(k), make_view<const QT>(v), make_view<QT>(*a.dk),
                          make_view<QT>(*a.dv), N, bs};
   if constexpr (DM > 0) {
-    sel_bwd_dkv_kernel<QT, DM, DenseGrad<QT>><<<static_cast<unsigned>(kv_items), kKvThreads, 0, s>>>(
-        make_view<const QT>(q), make_view<const QT>(*a.dout), kg, nl2, delta, offsets, groups, M,
-        H, G, MG, T, NS, nkt, ch, causal, a.scale, nsub);
+    return launch_dkv<QT, DM>(q, *a.dout, kg, nl2, delta, offsets, groups, M, H, G, MG, T, NS, bs,
+                              ch, causal, a.scale, s);
   } else {
     sel_bwd_dkv_valu_kernel<QT, DQ, DenseGrad<QT>><<<static_cast<unsigned>(kv_items), 256, 0, s>>>(
         make_view<const QT>(q), make_view<const QT>(*a.dout), kg, a.lse, delta, offsets, groups,
@@ -1176,9 +1238,8 @@ int sel_bwd_ptr_launch(const PtrBwdArgs& a, char* ws, const BwdWs& L, hipStream_
   rc = check_launch("pointer selection backward (index)");
   if (rc) return rc;
   if constexpr (DM > 0) {
-    sel_bwd_dkv_kernel<QT, DM, PtrGrad><<<static_cast<unsigned>(kv_items), kKvThreads, 0, s>>>(
-        make_view<const QT>(q), make_view<const QT>(*a.dout), a.kg, nl2, a.delta, offsets, groups,
-        M, H, G, MG, T, NS, nkt, 1, false, a.scale, nsub);
+    return launch_dkv<QT, DM>(q, *a.dout, a.kg, nl2, a.delta, offsets, groups, M, H, G, MG, T, NS,
+                              a.bs, 1, false, a.scale, s);
   } else {
     sel_bwd_dkv_valu_kernel<QT, DQ, PtrGrad><<<static_cast<unsigned>(kv_items), 256, 0, s>>>(
         make_view<const QT>(q), make_view<const QT>(*a.dout), a.kg, a.lse, a.delta, offsets,
@@ -1253,7 +1314,7 @@ extern "C" int omm_sel_bwd(const omm_view4* q, const omm_view4* k, const omm_vie
   bool rows_ok = true;
   for (const omm_view4* x : {q, k, v, out, dout, dq, dk, dv}) rows_ok = rows_ok && rows16(*x, D);
   const bool mfma = (dtype == OMM_BF16 || dtype == OMM_F16) && (D == 64 || D == 128) && rows_ok &&
-                    scale != 0.0f;
+                    scale != 0.0f && M < (int64_t{1} << 29);
   OMM_REQUIRE(mfma || k->stride[3] == v->stride[3], OMM_EUNSUPPORTED,
               "omm_sel_bwd: k and v need the same dim stride");
   char* ws = static_cast<char*>(workspace);
@@ -1367,7 +1428,8 @@ extern "C" int omm_sel_bwd_ptr(const omm_view4* q, const omm_view4* out, const f
   bool rows_ok = true;
   for (const omm_view4* x : {q, out, dout, dq}) rows_ok = rows_ok && rows16(*x, D);
   const bool mfma = (D == 64 || D == 128) && stride_bd == 1 && stride_bn % 8 == 0 &&
-                    2 * stride_bn * 64 < (int64_t{1} << 31) && rows_ok && scale != 0.0f;
+                    2 * stride_bn * 64 < (int64_t{1} << 31) && rows_ok && scale != 0.0f &&
+                    M < (int64_t{1} << 29);
   char* ws = static_cast<char*>(workspace);
   const hipStream_t s = static_cast<hipStream_t>(stream);
   if (mfma) return D == 128 ? sel_bwd_ptr_launch<128, 0>(a, ws, L, s) : sel_bwd_ptr_launch<64, 0>(a, ws, L, s);
