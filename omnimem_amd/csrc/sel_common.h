@@ -131,6 +131,7 @@ inline bool kv_offsets_fit32(const omm_view4& k, const omm_view4& v) {
 template <typename T>
 struct DenseAcc {
   static constexpr bool kMayMisalign = false;  // 16-byte rows checked on the host
+  static constexpr bool kHistory = false;
   using KV = T;
   struct Ent {
     int t0, n;  // first token, visible tokens
@@ -175,6 +176,7 @@ struct PtrAcc {
   // raw caller addresses: any 2-byte alignment is accepted (the reference's contract), so the
   // staging checks each block and copies misaligned ones with 2-byte loads
   static constexpr bool kMayMisalign = true;
+  static constexpr bool kHistory = true;  // blocks of a cache, as many as a long video's
   struct Ent {
     int64_t k, v;  // raw addresses (0 = skip)
     int n;
@@ -216,6 +218,7 @@ template <> struct PagedEntOf<uint8_t> { using type = PagedEnt8; };
 template <typename KVT>
 struct PagedAcc {
   static constexpr bool kMayMisalign = false;  // 16-byte rows checked on the host
+  static constexpr bool kHistory = true;  // blocks of a cache, as many as a long video's
   using KV = KVT;
   using Ent = typename PagedEntOf<KVT>::type;
   const KVT* pool_k;
@@ -589,6 +592,70 @@ __device__ __forceinline__ void copy_part(const void* base, int rsb, int nrows, 
   }
   dma_part<NI>(base, rsb, nrows, dst, w, off);
 }
+
+// ---- one-wave workgroups (query groups of at most 32) ----------------------------------------
+// A tile of 32 rows (keys) in a wave's own LDS buffer.  Two lane offsets and the row stride describe
+// its copy; what else a copy or an operand read needs is formed at each use (opaque keeps it
+// there), because held across the loop those offsets cost a wave per SIMD.
+__device__ __forceinline__ int opaque(int x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
+
+template <typename Acc, int D>
+struct WaveTile {
+  using DG = DmaGeom<D>;
+  static constexpr int TK = 32, NT = 2, SD = D / 32, ND = D / 16;
+  static constexpr int NI = TK / DG::RPI;  // copy instructions per tile (8 or 4)
+  static constexpr int BYTES = TK * DG::ROWB;
+  int c0, c1;  // this lane's source offsets of copy instructions 0 and (D = 128) 1
+  int rsb;     // row stride in bytes
+
+  __device__ __forceinline__ void init(int rs) {
+    const int lane = lane_id();
+    rsb = rs;
+    const int r0 = lane / DG::CPR, r1 = DG::RPI + r0, c = lane % DG::CPR;
+    c0 = r0 * rs + ((c ^ DG::swz_v(r0)) << 4);
+    c1 = r1 * rs + ((c ^ DG::swz_v(r1)) << 4);
+  }
+  // Rows [0, n) of a block from token tok on into dst; rows past n become 0.  The swizzle of a row
+  // depends on the row modulo 8, so instructions 8 rows apart differ by 8 row strides.
+  __device__ __forceinline__ void copy(const void* block, int tok, int n, char* dst) const {
+    constexpr int STEP = 8 / DG::RPI;  // instructions per 8 rows (2 or 1)
+    const char* base = static_cast<const char*>(block) + static_cast<int64_t>(tok) * rsb;
+    const int a0 = opaque(c0), a1 = STEP == 2 ? opaque(c1) : 0;
+#pragma unroll
+    for (int p = 0; p < NI / 4; ++p) {
+      int o[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int j = 4 * p + i;
+        o[i] = (STEP == 2 && (j & 1) ? a1 : a0) + (j / STEP) * 8 * rsb;
+      }
+      copy_part<Acc>(base, rsb, n, dst, p, o);
+    }
+  }
+  // Row operand (t, s): row 16 t + l16, dims 32 s + 8 j4 .. + 7.  r0 is this lane's offset of
+  // (0, 0); the step s flips bits of it.
+  __device__ __forceinline__ static int row0() {
+    const int l16 = lane_id() & 15, j4 = lane_id() >> 4;
+    return l16 * DG::ROWB + ((j4 ^ DG::swz_v(l16)) << 4);
+  }
+  __device__ __forceinline__ static uint4 row(const char* tile, int r0, int t, int s) {
+    return *reinterpret_cast<const uint4*>(tile + (r0 ^ (64 * s)) + 16 * t * DG::ROWB);
+  }
+  // Transposed operand i: dim 16 i + l16 of keys 4 j4 .. + 3 and 16 + 4 j4 .. + 3.  t0 is this
+  // lane's offset of dim tile 0; a dim tile flips bits of it (the swizzle is even).
+  __device__ __forceinline__ static int tr0() {
+    const int l16 = lane_id() & 15, vr = 4 * (lane_id() >> 4) + (l16 >> 2), vm = l16 & 3;
+    return vr * DG::ROWB + (((vm >> 1) ^ DG::swz_v(vr)) << 4) + ((vm & 1) << 3);
+  }
+  __device__ __forceinline__ static uint4 tr(const char* tile, int t0, int i) {
+    const char* p = tile + (t0 ^ (32 * i));
+    const uint2 lo = lds_read_tr16(p), hi = lds_read_tr16(p + 16 * DG::ROWB);
+    return make_uint4(lo.x, lo.y, hi.x, hi.y);
+  }
+};
 
 }  // namespace
 }  // namespace omm

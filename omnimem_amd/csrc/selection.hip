@@ -920,6 +920,237 @@ __global__ __launch_bounds__(NW * kWave, 2) void sel_fwd_dma_kernel(
   }
 }
 
+// ---- one-wave kernel (16-bit K / V, query groups of at most 32) ----------------------------------
+// One workgroup = one query group = one wave of QB 16-query row blocks, so a small group leaves no
+// wave and at most 15 rows without a query (the 64-query kernel above spends 49 of its rows on a
+// group of 15).  The group reads 16 KiB of K and V per 32 keys for 16 QB queries, and that stream is
+// what bounds the kernel: a CU takes at most 64 bytes a cycle of it, and of random selections over a
+// clip four bytes in ten miss L2 (6.2 TB/s of misses at the first size below; from 6 waves a CU on
+// their number makes no difference).  A tile's operands are read from LDS into registers first, the
+// next tile's copies are issued behind them into the same buffers, and S, softmax and P V of one wave
+// run under the copies of the others; there is no barrier.
+// 32760 tokens, 12 heads, top-16, blocks of 30, groups of 15: 450 us, 545 us with the 64-query
+// kernel (same ids for every group, all L2 hits: 279 and 526 us); groups of 30 and blocks of 60
+// 382 and 504 us; groups and blocks of 24, top-64 763 and 1150 us; head dim 64 (30 / 15) 166 and
+// 608 us.  K rows loaded from global memory straight into registers as operands (16 rows of 64
+// bytes an instruction, only V through LDS) took 522 us, whatever the number of waves (2 to 4).
+template <typename QT, typename Acc, int D, int QB>
+__global__ __launch_bounds__(kWave, 2) void sel_fwd_wave_kernel(
+    View4<const QT> q, View4<QT> out, float* __restrict__ lse, Acc acc, int M, int H, int G,
+    int MG, int T, int chunk, float scale, GateArgs gate, bool early) {
+  using WT = WaveTile<Acc, D>;
+  constexpr int TK = WT::TK, NT = WT::NT, SD = WT::SD, ND = WT::ND;
+  __shared__ __align__(16) char lds[2 * WT::BYTES];  // a K tile, a V tile
+
+  const int lane = lane_id(), l16 = lane & 15, j4 = lane >> 4;
+  int wi = xcd_remap(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x));
+  const int g = wi % MG; wi /= MG;
+  const int h = wi % H;
+  const int b = wi / H;
+  const int m0 = g * G, m_end = min(m0 + G, M);
+  const int qc = m0 / chunk;
+  acc.touch(b, g, h, T);
+
+  bool q_ok[QB];
+  uint4 qb[QB][SD];
+#pragma unroll
+  for (int x = 0; x < QB; ++x) {
+    const int mq = m0 + 16 * x + l16;
+    q_ok[x] = mq < m_end;
+#pragma unroll
+    for (int s = 0; s < SD; ++s)
+      qb[x][s] = q_ok[x] ? *reinterpret_cast<const uint4*>(q.at(b, mq, h, 32 * s + 8 * j4))
+                         : make_uint4(0, 0, 0, 0);
+  }
+  // the softmax works on s * c2 with c2 > 0; a negative scale negates Q instead, which is exact
+  float c2 = scale * kLog2e;
+  if (c2 < 0.0f) {
+    c2 = -c2;
+#pragma unroll
+    for (int x = 0; x < QB; ++x)
+#pragma unroll
+      for (int s = 0; s < SD; ++s) {
+        qb[x][s].x ^= 0x80008000u;
+        qb[x][s].y ^= 0x80008000u;
+        qb[x][s].z ^= 0x80008000u;
+        qb[x][s].w ^= 0x80008000u;
+      }
+  }
+  const int row0 = WT::row0(), tr0 = WT::tr0();
+
+  f32x4 o[QB][ND];
+#pragma unroll
+  for (int x = 0; x < QB; ++x)
+#pragma unroll
+    for (int i = 0; i < ND; ++i) o[x][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m2[QB], nms[QB], lsum[QB];
+#pragma unroll
+  for (int x = 0; x < QB; ++x) {
+    m2[x] = kNegInf;
+    nms[x] = lsum[x] = 0.0f;
+  }
+  bool started = false;  // every row of the wave has seen a visible key
+
+  WaveWalk<Acc, TK> wk;
+  wk.start(acc, b, g, h, T, qc);
+  WT kt, vt;
+  int n_cur = 0;  // visible keys of the current tile (0: done)
+  auto fetch = [&]() {
+    const int tok = __builtin_amdgcn_readfirstlane(wk.tok0);
+    kt.copy(wk.br.k, tok, wk.n, lds);
+    vt.copy(wk.br.v, tok, wk.n, lds + WT::BYTES);
+  };
+  if (wk.valid) {
+    // row strides are the same for every block of a call
+    kt.init(static_cast<int>(wk.br.sk) * 2);
+    vt.init(static_cast<int>(wk.br.sv) * 2);
+    fetch();
+    n_cur = wk.n;
+    wk.advance(acc, b, g, h, T, qc);
+  }
+  __builtin_amdgcn_s_waitcnt(0);  // Q, the walk's loads and the first tile's copies
+  while (n_cur > 0) {
+    // the tile's copies have landed; its operands leave the buffers for the next tile's
+    uint4 ka[NT][SD], va[ND];
+    const int r0 = opaque(row0), t0 = opaque(tr0);
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int s = 0; s < SD; ++s) ka[t][s] = WT::row(lds, r0, t, s);
+#pragma unroll
+    for (int i = 0; i < ND; ++i) va[i] = WT::tr(lds + WT::BYTES, t0, i);
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    int n_nx = 0;
+    if (wk.valid) {
+      fetch();
+      n_nx = wk.n;
+      wk.advance(acc, b, g, h, T, qc);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (early) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // launch-uniform
+    // S^T = K Q^T: lane holds keys 16 t + 4 j4 + r of query l16
+    f32x4 s4[QB][NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int x = 0; x < QB; ++x) {
+        s4[x][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < SD; ++s) s4[x][t] = Mfma<QT>::run(ka[t][s], qb[x][s], s4[x][t]);
+      }
+    if (n_cur < TK) {  // partial tile: keys past n_cur are not visible
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (16 * t + 4 * j4 + r >= n_cur) {
+#pragma unroll
+            for (int x = 0; x < QB; ++x) s4[x][t][r] = kNegInf;
+          }
+    }
+    // online softmax: the 64-query kernel's scheme (the running max moves before a row's first
+    // visible key and when a lane's sum of the tile's p for the row passes 256)
+#pragma unroll
+    for (int x = 0; x < QB; ++x) {
+      const float msafe = -nms[x];
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) s4[x][t][r] = __builtin_fmaf(s4[x][t][r], c2, -msafe);
+    }
+    auto move_max = [&]() {
+#pragma unroll
+      for (int x = 0; x < QB; ++x) {
+        const float msafe = m2[x] == kNegInf ? 0.0f : m2[x];
+        float v = kNegInf;
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+          v = fmaxf(v, fmaxf(fmaxf(s4[x][t][0], s4[x][t][1]), fmaxf(s4[x][t][2], s4[x][t][3])));
+        v = fmaxf(v, __shfl_xor(v, 16, kWave));
+        v = fmaxf(v, __shfl_xor(v, 32, kWave));
+        const float mcand = fmaxf(m2[x], v + msafe);
+        const float msafe_new = mcand == kNegInf ? 0.0f : mcand;
+        const float alpha = __builtin_amdgcn_exp2f(m2[x] - msafe_new);
+        lsum[x] *= alpha;
+#pragma unroll
+        for (int i = 0; i < ND; ++i) o[x][i] *= alpha;
+        m2[x] = mcand;
+        nms[x] = -msafe_new;
+        const float shift = msafe - msafe_new;
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) s4[x][t][r] += shift;
+      }
+    };
+    if (!started) {  // wave-uniform
+      move_max();
+      bool any = false;
+#pragma unroll
+      for (int x = 0; x < QB; ++x) any = any || m2[x] == kNegInf;
+      started = __ballot(any) == 0ull;
+    }
+    uint4 pb[QB];
+    float ps[QB];
+    auto exps = [&]() {
+#pragma unroll
+      for (int x = 0; x < QB; ++x) {
+        float pv[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) pv[e] = __builtin_amdgcn_exp2f(s4[x][e >> 2][e & 3]);
+        ps[x] = ((pv[0] + pv[1]) + (pv[2] + pv[3])) + ((pv[4] + pv[5]) + (pv[6] + pv[7]));
+        pb[x] = make_uint4(Mfma<QT>::pack2(pv[0], pv[1]), Mfma<QT>::pack2(pv[2], pv[3]),
+                           Mfma<QT>::pack2(pv[4], pv[5]), Mfma<QT>::pack2(pv[6], pv[7]));
+      }
+    };
+    exps();
+    bool over = false;
+#pragma unroll
+    for (int x = 0; x < QB; ++x) over = over || ps[x] > 256.0f;
+    if (__ballot(over) != 0ull) {
+      move_max();
+      exps();
+    }
+#pragma unroll
+    for (int x = 0; x < QB; ++x) lsum[x] += ps[x];
+    // O^T += V^T P^T
+#pragma unroll
+    for (int i = 0; i < ND; ++i)
+#pragma unroll
+      for (int x = 0; x < QB; ++x) o[x][i] = Mfma<QT>::run(va[i], pb[x], o[x][i]);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the next tile's copies
+    n_cur = n_nx;
+  }
+
+#pragma unroll
+  for (int x = 0; x < QB; ++x) {
+    float ls = lsum[x];
+    ls += __shfl_xor(ls, 16, kWave);
+    ls += __shfl_xor(ls, 32, kWave);
+    if (!q_ok[x]) continue;
+    const int mq = m0 + 16 * x + l16;
+    const float inv = ls > 0.0f ? 1.0f / ls : 0.0f;
+    QT* op = out.at(b, mq, h, 0);
+#pragma unroll
+    for (int i = 0; i < ND; ++i) {
+      uint2 w2;
+      if (gate.g != nullptr) {  // launch-uniform
+        const float o4[4] = {o[x][i][0] * inv, o[x][i][1] * inv, o[x][i][2] * inv,
+                             o[x][i][3] * inv};
+        w2 = gate_mix4(gate, b, mq, h, 16 * i + 4 * j4, o4);
+      } else {
+        w2.x = Mfma<QT>::pack2(o[x][i][0] * inv, o[x][i][1] * inv);
+        w2.y = Mfma<QT>::pack2(o[x][i][2] * inv, o[x][i][3] * inv);
+      }
+      *reinterpret_cast<uint2*>(op + 16 * i + 4 * j4) = w2;
+    }
+    if (lse != nullptr && j4 == 0)
+      lse[(static_cast<int64_t>(b) * H + h) * M + mq] =
+          ls > 0.0f ? (m2[x] + __builtin_log2f(ls)) * kLn2 : kNegInf;
+  }
+}
+
 // ---- fp32 MFMA kernel (fp32 q / k / v, head dim 64 or 128) ---------------------------------------
 // One workgroup = one query group of up to 64 queries, 4 waves x 16 queries (the fp32 MFMA is
 // 32 cycles long, so one operand read per MFMA costs little, and 16-query waves give config 1's
@@ -1455,22 +1686,6 @@ int launch_qk8(const Geom& gm, const omm_view4& q, const omm_view4& out, float* 
   return rc;
 }
 
-template <typename QT, typename Acc, int D>
-int launch_dma(const Geom& gm, const omm_view4& q, const omm_view4& out, float* lse,
-               const Acc& acc, int chunk, float scale, hipStream_t s, const GateArgs& gate) {
-  if (gm.nsub >= 2) {  // two 64-query subgroups per workgroup
-    const int64_t grid = gm.items / gm.nsub * ((gm.nsub + 1) / 2);
-    sel_fwd_dma_kernel<QT, Acc, D, 4><<<static_cast<unsigned>(grid), 4 * kWave, 0, s>>>(
-        make_view<const QT>(q), make_view<QT>(out), lse, acc, gm.M, gm.H, gm.G, gm.MG, gm.T,
-        chunk, scale, gm.nsub, gate);
-  } else {
-    sel_fwd_dma_kernel<QT, Acc, D, 2><<<static_cast<unsigned>(gm.items), 2 * kWave, 0, s>>>(
-        make_view<const QT>(q), make_view<QT>(out), lse, acc, gm.M, gm.H, gm.G, gm.MG, gm.T,
-        chunk, scale, gm.nsub, gate);
-  }
-  return check_launch("selection attention (dma)");
-}
-
 // Compute units of the current device (0 when the runtime cannot say), cached per device.
 inline int device_cus() {
   static std::atomic<int> cache[64];
@@ -1483,6 +1698,54 @@ inline int device_cus() {
     cache[dev].store(n, std::memory_order_relaxed);
   }
   return n;
+}
+
+// Whether one wave per query group takes a call (sel_fwd_wave_kernel).  A cache call of groups of 17
+// to 32 queries with at most 8 of them per CU keeps the 64-query kernel, which has two tiles in
+// flight: 30-query groups over 60-token blocks, 7.3 per CU, 135.0 against 137.3 us.
+template <typename Acc>
+bool wave_kernel(const Geom& gm) {
+  return gm.G <= 16 ||
+         (gm.G <= 32 && !(Acc::kHistory && gm.items <= int64_t{8} * device_cus()));
+}
+
+template <typename QT, typename Acc, int D>
+int launch_dma(const Geom& gm, const omm_view4& q, const omm_view4& out, float* lse,
+               const Acc& acc, int chunk, float scale, hipStream_t s, const GateArgs& gate) {
+  if (wave_kernel<Acc>(gm)) {
+    // A cache's blocks do not fit the memory-side cache, and the fewer groups sweep them at a time
+    // the more of them share a block: 6 waves a CU (by LDS) where the call has more than 8 for
+    // each.  Over 27 chunks of 4680 tokens, 12 heads, top-16: 142 us with 10, 134 with 6, 139 with
+    // the 64-query kernel; top-64 over blocks and groups of 24 262, 225 and 265 us.  (Of a clip,
+    // which fits, more waves are better: 458 us with 6, 450 with 10; head dim 64 196 and 165.)
+    const bool few = Acc::kHistory && gm.items > int64_t{8} * device_cus();
+    const size_t lds = few ? 27000 - 2 * WaveTile<Acc, D>::BYTES : 0;
+    // Waiting for the next tile's copies before this tile's S keeps fewer in flight, which short
+    // lists over a clip share better in L2: blocks of 30, groups of 15 450 us, waiting at the end
+    // 458 (16380 tokens 160 and 167; 60 / 30 384 and 400).  Long lists and caches wait at the end:
+    // top-64 over 24 / 24 735 us against 752 (4680 tokens 147 and 157; a cache of 27 chunks 225
+    // and 242).
+    const bool early = !Acc::kHistory && gm.T <= 32;
+    const unsigned grid = static_cast<unsigned>(gm.items);
+    if (gm.G <= 16)
+      sel_fwd_wave_kernel<QT, Acc, D, 1><<<grid, kWave, lds, s>>>(
+          make_view<const QT>(q), make_view<QT>(out), lse, acc, gm.M, gm.H, gm.G, gm.MG, gm.T,
+          chunk, scale, gate, early);
+    else
+      sel_fwd_wave_kernel<QT, Acc, D, 2><<<grid, kWave, lds, s>>>(
+          make_view<const QT>(q), make_view<QT>(out), lse, acc, gm.M, gm.H, gm.G, gm.MG, gm.T,
+          chunk, scale, gate, early);
+  } else if (gm.nsub >= 2) {  // two 64-query subgroups per workgroup
+    const int64_t grid = gm.items / gm.nsub * ((gm.nsub + 1) / 2);
+    sel_fwd_dma_kernel<QT, Acc, D, 4><<<static_cast<unsigned>(grid), 4 * kWave, 0, s>>>(
+        make_view<const QT>(q), make_view<QT>(out), lse, acc, gm.M, gm.H, gm.G, gm.MG, gm.T,
+        chunk, scale, gm.nsub, gate);
+  } else {
+    sel_fwd_dma_kernel<QT, Acc, D, 2><<<static_cast<unsigned>(gm.items), 2 * kWave, 0, s>>>(
+        make_view<const QT>(q), make_view<QT>(out), lse, acc, gm.M, gm.H, gm.G, gm.MG, gm.T,
+        chunk, scale, gm.nsub, gate);
+  }
+  return check_launch("selection attention (dma)");
 }
 
 // A split fp32 call runs kF32RunsPerCu equal runs per CU when it has fewer than kF32SplitBelow

@@ -82,6 +82,30 @@ def test_sel_fwd_matches_oracle(dtype, case):
     _check(out, lse, want_o, want_l, dtype)
 
 
+@pytest.mark.parametrize("BS", [16, 30, 32, 33, 64, 65])
+@pytest.mark.parametrize("G", [1, 15, 16, 17, 31, 32, 33])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("scale", [None, -0.2])
+def test_sel_fwd_small_group_edges(BS, G, D, scale):
+    """Groups around the sizes where one wave with one or two 16-query row blocks takes a group (16,
+    32), over blocks that fill, split and do not fill its 32-key tiles, with rows that see nothing
+    at first, -1 ids, more slots than the walk resolves at once (64) and a negative scale."""
+    from omnimem_amd.selection import sel_fwd
+    M, N, H, T, chunk = 100, 333, 2, 67 if BS == 16 else 5, 60
+    gen = torch.Generator().manual_seed(BS * 100 + G)
+    q = (torch.randn((1, M, H, D), generator=gen) * D ** -0.25).bfloat16()
+    k = (torch.randn((1, N, H, D), generator=gen) * D ** -0.25).bfloat16()
+    v = torch.randn((1, N, H, D), generator=gen).bfloat16()
+    ids = _ids(gen, 1, -(-M // G), H, T, -(-N // BS) + 1, 0.2)
+    sc = D ** -0.5 if scale is None else scale
+    out, lse = sel_fwd(q.to(DEV), k.to(DEV), v.to(DEV), ids.to(DEV), BS, chunk, sc, True, G)
+    want_o, want_l = O.selection_attention(q.float().numpy(), k.float().numpy(), v.float().numpy(),
+                                           ids.numpy(), G, sc,
+                                           O.dense_block_tokens(N, BS, chunk, True),
+                                           chunk_size=chunk, causal=True)
+    _check(out, lse, want_o, want_l, torch.bfloat16)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("scale", [-0.09, 0.0, 8.0])
 def test_sel_fwd_scale_values(scale, dtype):
