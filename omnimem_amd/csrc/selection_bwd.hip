@@ -282,6 +282,198 @@ __global__ __launch_bounds__(kDqThreads, 2) void sel_bwd_dq_kernel(
   }
 }
 
+// One wave per query group of at most 32 (QB 16-query row blocks), tiles of 32 keys: the forward's
+// one-wave kernel with dO beside Q.  The K and V tiles are read from LDS as rows, K also transposed;
+// all of a tile's operands are in registers before its buffers take the next tile.  The whole
+// backward of 32760 tokens, 12 heads, top-16 with the 64-query kernel and with this one: blocks of 30
+// and groups of 15 1114 and 967 us (head dim 64 964 and 482 us), 60 / 30 1248 and 1075 us, top-64
+// over blocks and groups of 24 3150 and 2513 us.
+template <typename QT, typename Acc, int D, int QB>
+__global__ __launch_bounds__(kWave, 2) void sel_bwd_dq_wave_kernel(
+    View4<const QT> q, View4<const QT> o, View4<const QT> dout, View4<QT> dq,
+    const float* __restrict__ lse, float* __restrict__ delta, float* __restrict__ nl2out, Acc acc,
+    int M, int H, int G, int MG, int T, int chunk, float scale) {
+  using WT = WaveTile<Acc, D>;
+  constexpr int TK = WT::TK, NT = WT::NT, SD = WT::SD, ND = WT::ND;
+  __shared__ __align__(16) char lds[2 * WT::BYTES];  // a K tile, a V tile
+
+  const int lane = lane_id(), l16 = lane & 15, j4 = lane >> 4;
+  int wi = xcd_remap(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x));
+  const int g = wi % MG; wi /= MG;
+  const int h = wi % H;
+  const int b = wi / H;
+  const int m0 = g * G, m_end = min(m0 + G, M);
+  const int qc = m0 / chunk;
+
+  // Q^T and dO^T operands, each query's delta (a 4-lane-group reduction) and -lse log2 e
+  bool q_ok[QB];
+  uint4 qb[QB][SD], db[QB][SD];
+  float nl2[QB], dl[QB];
+#pragma unroll
+  for (int x = 0; x < QB; ++x) {
+    const int mq = m0 + 16 * x + l16;
+    q_ok[x] = mq < m_end;
+    float part = 0.0f;
+#pragma unroll
+    for (int s = 0; s < SD; ++s) {
+      if (q_ok[x]) {
+        qb[x][s] = *reinterpret_cast<const uint4*>(q.at(b, mq, h, 32 * s + 8 * j4));
+        db[x][s] = *reinterpret_cast<const uint4*>(dout.at(b, mq, h, 32 * s + 8 * j4));
+        part += dot8<QT>(*reinterpret_cast<const uint4*>(o.at(b, mq, h, 32 * s + 8 * j4)),
+                         db[x][s]);
+      } else {
+        qb[x][s] = make_uint4(0, 0, 0, 0);
+        db[x][s] = make_uint4(0, 0, 0, 0);
+      }
+    }
+    part += __shfl_xor(part, 16, kWave);
+    part += __shfl_xor(part, 32, kWave);
+    dl[x] = part;
+    const int64_t li = (static_cast<int64_t>(b) * H + h) * M + mq;
+    nl2[x] = q_ok[x] ? neg_lse2(lse[li]) : kNegInf;
+    if (q_ok[x] && j4 == 0) {
+      delta[li] = part;
+      nl2out[li] = nl2[x];
+    }
+  }
+  const float c2 = scale * kLog2e;
+  // dO^T negated (exact) and delta as the accumulator input, as in the kernel above
+#pragma unroll
+  for (int x = 0; x < QB; ++x)
+#pragma unroll
+    for (int s = 0; s < SD; ++s) {
+      db[x][s].x ^= 0x80008000u;
+      db[x][s].y ^= 0x80008000u;
+      db[x][s].z ^= 0x80008000u;
+      db[x][s].w ^= 0x80008000u;
+    }
+  const int row0 = WT::row0(), tr0 = WT::tr0();
+  f32x4 acc_dq[QB][ND];
+#pragma unroll
+  for (int x = 0; x < QB; ++x)
+#pragma unroll
+    for (int i = 0; i < ND; ++i) acc_dq[x][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  WaveWalk<Acc, TK> wk;
+  wk.start(acc, b, g, h, T, qc);
+  WT kt, vt;
+  int n_cur = 0;
+  auto fetch = [&]() {
+    const int tok = __builtin_amdgcn_readfirstlane(wk.tok0);
+    kt.copy(wk.br.k, tok, wk.n, lds);
+    vt.copy(wk.br.v, tok, wk.n, lds + WT::BYTES);
+  };
+  if (wk.valid) {
+    kt.init(static_cast<int>(wk.br.sk) * 2);
+    vt.init(static_cast<int>(wk.br.sv) * 2);
+    fetch();
+    n_cur = wk.n;
+    wk.advance(acc, b, g, h, T, qc);
+  }
+  __builtin_amdgcn_s_waitcnt(0);
+  while (n_cur > 0) {
+    // S^T = K Q^T and dP^T - delta (negated): lane holds keys 16 t + 4 j4 + r of query l16
+    const int r0 = opaque(row0), t0 = opaque(tr0);
+    f32x4 s4[QB][NT], p4[QB][NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+#pragma unroll
+      for (int x = 0; x < QB; ++x) {
+        s4[x][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        p4[x][t] = f32x4{dl[x], dl[x], dl[x], dl[x]};
+      }
+#pragma unroll
+      for (int s = 0; s < SD; ++s) {
+        const uint4 ka = WT::row(lds, r0, t, s), va = WT::row(lds + WT::BYTES, r0, t, s);
+#pragma unroll
+        for (int x = 0; x < QB; ++x) {
+          s4[x][t] = Mfma<QT>::run(ka, qb[x][s], s4[x][t]);
+          p4[x][t] = Mfma<QT>::run(va, db[x][s], p4[x][t]);
+        }
+      }
+    }
+    uint4 kt4[ND];
+#pragma unroll
+    for (int i = 0; i < ND; ++i) kt4[i] = WT::tr(lds, t0, i);
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    int n_nx = 0;
+    if (wk.valid) {
+      fetch();
+      n_nx = wk.n;
+      wk.advance(acc, b, g, h, T, qc);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // dS / scale = P (dP - delta), P = 2^e, e = s c2 - lse log2 e; e = -inf past the visible keys
+#pragma unroll
+    for (int x = 0; x < QB; ++x)
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) s4[x][t][r] = __builtin_fmaf(s4[x][t][r], c2, nl2[x]);
+    if (n_cur < TK) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (16 * t + 4 * j4 + r >= n_cur) {
+#pragma unroll
+            for (int x = 0; x < QB; ++x) s4[x][t][r] = kNegInf;
+          }
+    }
+    // dQ^T += K^T dS^T
+    uint4 sb[QB];
+#pragma unroll
+    for (int x = 0; x < QB; ++x) {
+      float d[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        d[e] = -(__builtin_amdgcn_exp2f(s4[x][e >> 2][e & 3]) * p4[x][e >> 2][e & 3]);
+      sb[x] = make_uint4(Mfma<QT>::pack2(d[0], d[1]), Mfma<QT>::pack2(d[2], d[3]),
+                         Mfma<QT>::pack2(d[4], d[5]), Mfma<QT>::pack2(d[6], d[7]));
+    }
+#pragma unroll
+    for (int i = 0; i < ND; ++i)
+#pragma unroll
+      for (int x = 0; x < QB; ++x) acc_dq[x][i] = Mfma<QT>::run(kt4[i], sb[x], acc_dq[x][i]);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the next tile's copies
+    n_cur = n_nx;
+  }
+
+#pragma unroll
+  for (int x = 0; x < QB; ++x) {
+    if (!q_ok[x]) continue;
+    QT* op = dq.at(b, m0 + 16 * x + l16, h, 0);
+#pragma unroll
+    for (int i = 0; i < ND; ++i) {
+      uint2 w2;
+      w2.x = Mfma<QT>::pack2(acc_dq[x][i][0] * scale, acc_dq[x][i][1] * scale);
+      w2.y = Mfma<QT>::pack2(acc_dq[x][i][2] * scale, acc_dq[x][i][3] * scale);
+      *reinterpret_cast<uint2*>(op + 16 * i + 4 * j4) = w2;
+    }
+  }
+}
+
+// The dQ kernel for a call's group size (MFMA paths).
+template <typename QT, typename Acc, int D>
+void launch_dq(const omm_view4& q, const omm_view4& out, const omm_view4& dout, const omm_view4& dq,
+               const float* lse, float* delta, float* nl2, const Acc& acc, int M, int H, int G,
+               int MG, int T, int chunk, float scale, int nsub, int64_t items, hipStream_t s) {
+  const unsigned grid = static_cast<unsigned>(items);
+  const auto qv = make_view<const QT>(q), ov = make_view<const QT>(out);
+  const auto dov = make_view<const QT>(dout);
+  const auto dqv = make_view<QT>(dq);
+  if (G <= 16)
+    sel_bwd_dq_wave_kernel<QT, Acc, D, 1><<<grid, kWave, 0, s>>>(
+        qv, ov, dov, dqv, lse, delta, nl2, acc, M, H, G, MG, T, chunk, scale);
+  else if (G <= 32)
+    sel_bwd_dq_wave_kernel<QT, Acc, D, 2><<<grid, kWave, 0, s>>>(
+        qv, ov, dov, dqv, lse, delta, nl2, acc, M, H, G, MG, T, chunk, scale);
+  else
+    sel_bwd_dq_kernel<QT, Acc, D><<<grid, kDqThreads, 0, s>>>(
+        qv, ov, dov, dqv, lse, delta, nl2, acc, M, H, G, MG, T, chunk, scale, nsub);
+}
+
 // ---- block -> query-group index --------------------------------------------------------------
 constexpr int kIdxThreads = 512;
 constexpr int kIdxWaves = kIdxThreads / kWave;
@@ -1152,9 +1344,8 @@ int sel_bwd_launch(const BwdArgs& a, char* ws, const BwdWs& L, hipStream_t s) {
   OMM_REQUIRE(dq_items <= 2147483647ll && kv_items <= 2147483647ll, OMM_EUNSUPPORTED,
               "omm_sel_bwd: grid too large");
   if constexpr (DM > 0) {
-    sel_bwd_dq_kernel<QT, DenseAcc<QT>, DM><<<static_cast<unsigned>(dq_items), kDqThreads, 0, s>>>(
-        make_view<const QT>(q), make_view<const QT>(*a.out), make_view<const QT>(*a.dout),
-        make_view<QT>(*a.dq), a.lse, delta, nl2, acc, M, H, G, MG, T, ch, a.scale, nsub);
+    launch_dq<QT, DenseAcc<QT>, DM>(q, *a.out, *a.dout, *a.dq, a.lse, delta, nl2, acc, M, H, G, MG,
+                                    T, ch, a.scale, nsub, dq_items, s);
   } else {
     sel_bwd_dq_valu_kernel<QT, DenseAcc<QT>, DQ><<<static_cast<unsigned>(dq_items), 256, 0, s>>>(
         make_view<const QT>(q), make_view<const QT>(*a.out), make_view<const QT>(*a.dout),
@@ -1218,9 +1409,8 @@ int sel_bwd_ptr_launch(const PtrBwdArgs& a, char* ws, const BwdWs& L, hipStream_
   OMM_REQUIRE(dq_items <= 2147483647ll && kv_items <= 2147483647ll, OMM_EUNSUPPORTED,
               "omm_sel_bwd_ptr: grid too large");
   if constexpr (DM > 0) {
-    sel_bwd_dq_kernel<QT, PtrAcc, DM><<<static_cast<unsigned>(dq_items), kDqThreads, 0, s>>>(
-        make_view<const QT>(q), make_view<const QT>(*a.out), make_view<const QT>(*a.dout),
-        make_view<QT>(*a.dq), a.lse, a.delta, nl2, a.acc, M, H, G, MG, T, 1, a.scale, nsub);
+    launch_dq<QT, PtrAcc, DM>(q, *a.out, *a.dout, *a.dq, a.lse, a.delta, nl2, a.acc, M, H, G, MG, T,
+                              1, a.scale, nsub, dq_items, s);
   } else {
     sel_bwd_dq_valu_kernel<QT, PtrAcc, DQ><<<static_cast<unsigned>(dq_items), 256, 0, s>>>(
         make_view<const QT>(q), make_view<const QT>(*a.out), make_view<const QT>(*a.dout),
