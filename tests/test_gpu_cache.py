@@ -1069,3 +1069,45 @@ def test_async_flush_pending_moves_with_snapshots_reset_and_evict_all():
     assert cache._moves is None and all(nc == 0 for nc in cache.n_chunks)
     _slots_balance(cache)
     cache.close()
+
+
+@pytest.mark.parametrize("n_chunks", [3, 32, 33])
+@pytest.mark.parametrize("G,T", [(15, 16), (64, 70)])
+def test_selection_counters_match_the_listings(n_chunks, G, T):
+    """Stamps, page reads, unit accesses and seen pages of two calls, with listings merged per unit
+    (up to 32 chunks) and one by one, rows longer than a wave, duplicates, -1 and unwritten ids."""
+    from omnimem_amd.block_cache import PagedKVCache
+    H, D, P, C, M = 3, 64, 16, 48, 150
+    ppc = C // P
+    cache = PagedKVCache(1, H, D, max_chunks=n_chunks + 1, chunk_len=C, page_tokens=P,
+                         window_chunks=0)
+    g = torch.Generator().manual_seed(n_chunks + G)
+    kv = torch.randn((1, C, H, D), generator=g).bfloat16().cuda()
+    for c in range(n_chunks):
+        cache.append(0, kv, kv, c)
+    q = torch.randn((1, M, H, D), generator=g).bfloat16().cuda()
+    before = cache.stamp[0].cpu().numpy().copy()
+    reads = np.zeros((H, n_chunks + 1), dtype=np.int64)
+    calls = np.zeros_like(reads)
+    seen = np.zeros((H, n_chunks + 1, ppc), dtype=np.uint8)
+    for call in range(2):
+        ids = torch.randint(-1, (n_chunks + 1) * ppc, (1, -(-M // G), H, T), generator=g,
+                            dtype=torch.int32)
+        if call:
+            ids[ids // ppc == 1] = -1  # chunk 1 keeps the first call's stamp
+        cache.select(q, ids.cuda(), 0, G)
+        epoch = cache._epoch
+        hit = np.zeros((H, n_chunks + 1), dtype=bool)
+        for h in range(H):
+            x = ids[0, :, h].numpy().ravel()
+            x = x[(x >= 0) & (x // ppc < n_chunks)]
+            np.add.at(reads[h], x // ppc, 1)
+            seen[h, x // ppc, x % ppc] = 1
+            hit[h, np.unique(x // ppc)] = True
+        calls += hit
+        before[hit] = epoch
+    np.testing.assert_array_equal(cache.stamp[0].cpu().numpy(), before)
+    np.testing.assert_array_equal(cache.reads[0].cpu().numpy(), reads)
+    np.testing.assert_array_equal(cache.touches[0].cpu().numpy(), calls)
+    np.testing.assert_array_equal(cache.seen[0].cpu().numpy(), seen)
+    cache.close()
