@@ -9,7 +9,7 @@
 // per-token chunk-causal prefix), :1329-1407 (dK / dV of never-selected tokens are 0, results
 // in the K / V dtype).
 //
-// gfx950 design (bf16 / f16), three launches:
+// gfx950 design (bf16 / f16; fp32 in the same three launches on its own MFMA kernels):
 //   sel_bwd_dq_kernel    one workgroup = 64 queries of one group, 2 waves x 32 queries, the same
 //                        block walk and LDS-DMA K / V tiles as the forward kernel.  Per key tile:
 //                        S^T = K Q^T and dP^T = V dO^T (K and V rows from LDS, Q^T and dO^T held
@@ -1039,6 +1039,349 @@ __global__ __launch_bounds__(NW * kWave, 2) void sel_bwd_dkv_kernel(
   }
 }
 
+// ---- fp32 MFMA kernels (fp32 rows of 16-byte alignment, head dim 64 or 128) --------------------
+// fp32 operands and fp32 accumulation on v_mfma_f32_16x16x4_f32 (32 cycles each), P and dS not
+// rounded.  Rows are handled 16 at a time: 16-byte chunk c of row r of a 16-row LDS tile sits at
+// chunk c ^ r, which keeps both kinds of operand read off each other's banks: row operands (row
+// l16, chunk 4 u + j4: the dims 16 u + 4 j4 + e of the k-steps 4 u + e, four of them a read) and
+// transposed ones (rows 4 j4 + r, dim 16 i + l16, one a read).  Against the VALU kernels, which
+// reread every LDS operand for each of 4 lanes and had one workgroup per query group: 1560 queries
+// over 16 blocks of 64 of 4680 keys, 12 heads, head dim 128: dQ 2171 -> 190 us, dK / dV 763 -> 248 us (94
+// and 125 us at the fp32 matrix rate); 3900 tokens over themselves 5560 -> 982 us for the whole
+// backward, with blocks of 30 and groups of 15 7900 -> 560.
+template <int D>
+struct F32Tile {
+  static constexpr int ROWB = 4 * D, CPR = D / 4, RPI = 1024 / ROWB;
+  static constexpr int NI = 16 / RPI;  // copy instructions per 16 rows (8 or 4)
+  static constexpr int BYTES = 16 * ROWB;
+  static constexpr int DU = D / 16;
+  // this lane's source offset in copy instruction j (rows of rs bytes)
+  __device__ __forceinline__ static int src(int j, int rs) {
+    const int row = j * RPI + lane_id() / CPR;
+    return row * rs + (((lane_id() % CPR) ^ row) << 4);
+  }
+  // byte offsets of row operand u = rb ^ (u << 6) and transposed operand (r, i) = tb[r] ^ (i << 6)
+  __device__ __forceinline__ static int rb() {
+    const int l16 = lane_id() & 15, j4 = lane_id() >> 4;
+    return l16 * ROWB + ((j4 ^ l16) << 4);
+  }
+  __device__ __forceinline__ static int tb(int r) {
+    const int l16 = lane_id() & 15, j4 = lane_id() >> 4;
+    return (4 * j4 + r) * ROWB + (j4 << 6) + (((l16 >> 2) ^ r) << 4) + ((l16 & 3) << 2);
+  }
+};
+
+__device__ __forceinline__ f32x4 mfma4(const float4& a, const float4& b, f32x4 c) {
+  c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b.x, c, 0, 0, 0);
+  c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b.y, c, 0, 0, 0);
+  c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, b.z, c, 0, 0, 0);
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b.w, c, 0, 0, 0);
+}
+
+// dQ (and delta, -lse log2 e) of 16 queries of one group: 4 waves that take every fourth 16-key tile
+// of the group's blocks, each in its own LDS buffers, so that a call of a few hundred groups fills
+// the CUs; their sums are added in wave order at the end.
+template <typename Acc, int D>
+__global__ __launch_bounds__(256, 2) void sel_bwd_dq_f32_kernel(
+    View4<const float> q, View4<const float> o, View4<const float> dout, View4<float> dq,
+    const float* __restrict__ lse, float* __restrict__ delta, float* __restrict__ nl2out, Acc acc,
+    int M, int H, int G, int MG, int T, int chunk, float scale, int nsub) {
+  using FT = F32Tile<D>;
+  constexpr int DU = FT::DU, NI = FT::NI;
+  __shared__ __align__(16) char smem[4][2][FT::BYTES];  // per wave: a K tile, a V tile
+  const int tid = static_cast<int>(threadIdx.x), lane = lane_id();
+  const int w = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int l16 = lane & 15, j4 = lane >> 4;
+  int wi = xcd_remap(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x));
+  const int sub = wi % nsub; wi /= nsub;
+  const int g = wi % MG; wi /= MG;
+  const int h = wi % H;
+  const int b = wi / H;
+  const int m0 = g * G + 16 * sub, m_end = min(min(g * G + G, M), m0 + 16);
+  const int qc = (g * G) / chunk;
+  if (m0 >= m_end) return;  // a ragged last group (workgroup-uniform)
+
+  // Q^T and dO^T operands: query l16, dims 16 u + 4 j4 + e
+  const int mq = m0 + l16;
+  const bool q_ok = mq < m_end;
+  float4 qf[DU], df[DU];
+  float dl = 0.0f;
+#pragma unroll
+  for (int u = 0; u < DU; ++u) {
+    qf[u] = df[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (q_ok) {
+      qf[u] = *reinterpret_cast<const float4*>(q.at(b, mq, h, 16 * u + 4 * j4));
+      df[u] = *reinterpret_cast<const float4*>(dout.at(b, mq, h, 16 * u + 4 * j4));
+      const float4 of = *reinterpret_cast<const float4*>(o.at(b, mq, h, 16 * u + 4 * j4));
+      dl += (of.x * df[u].x + of.y * df[u].y) + (of.z * df[u].z + of.w * df[u].w);
+    }
+  }
+  dl += __shfl_xor(dl, 16, kWave);
+  dl += __shfl_xor(dl, 32, kWave);
+  const int64_t li = (static_cast<int64_t>(b) * H + h) * M + mq;
+  const float nl2 = q_ok ? neg_lse2(lse[li]) : kNegInf;
+  if (w == 0 && q_ok && j4 == 0) {
+    delta[li] = dl;
+    nl2out[li] = nl2;
+  }
+  const float c2 = scale * kLog2e;
+  const int rb = FT::rb();
+  int tb[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) tb[r] = FT::tb(r);
+  f32x4 acc_dq[DU];
+#pragma unroll
+  for (int i = 0; i < DU; ++i) acc_dq[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  char* const kbuf = smem[w][0];
+  char* const vbuf = smem[w][1];
+  WaveWalk<Acc, 16> wk;
+  wk.start(acc, b, g, h, T, qc);
+  auto skip = [&](int n) {
+    for (int i = 0; i < n && wk.valid; ++i) wk.advance(acc, b, g, h, T, qc);
+  };
+  skip(w);
+  int ko[NI], vo[NI], rsk = 0, rsv = 0;
+  auto fetch = [&](const void* block, int rs, const int (&off)[NI], char* dst) {
+    const char* base = static_cast<const char*>(block) +
+                       static_cast<int64_t>(__builtin_amdgcn_readfirstlane(wk.tok0)) * rs;
+#pragma unroll
+    for (int p = 0; p < NI / 4; ++p) {
+      const int o4[4] = {off[4 * p], off[4 * p + 1], off[4 * p + 2], off[4 * p + 3]};
+      dma_part<4>(base, rs, wk.n, dst, p, o4);
+    }
+  };
+  if (wk.valid) {
+    rsk = static_cast<int>(wk.br.sk) * 4;
+    rsv = static_cast<int>(wk.br.sv) * 4;
+#pragma unroll
+    for (int j = 0; j < NI; ++j) {
+      ko[j] = FT::src(j, rsk);
+      vo[j] = FT::src(j, rsv);
+    }
+    fetch(wk.br.k, rsk, ko, kbuf);
+    fetch(wk.br.v, rsv, vo, vbuf);
+  }
+  __builtin_amdgcn_s_waitcnt(0);
+  while (wk.valid) {
+    const int n = wk.n;
+    // S^T = K Q^T and dP^T = V dO^T: lane holds keys 4 j4 + r of query l16
+    f32x4 s4 = f32x4{0.f, 0.f, 0.f, 0.f}, p4 = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < DU; ++u)
+      s4 = mfma4(*reinterpret_cast<const float4*>(kbuf + (rb ^ (u << 6))), qf[u], s4);
+#pragma unroll
+    for (int u = 0; u < DU; ++u)
+      p4 = mfma4(*reinterpret_cast<const float4*>(vbuf + (rb ^ (u << 6))), df[u], p4);
+    // dS / scale = P (dP - delta); keys past n are not visible
+    float ds[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float p = 4 * j4 + r < n ? __builtin_amdgcn_exp2f(__builtin_fmaf(s4[r], c2, nl2)) : 0.0f;
+      ds[r] = p * (p4[r] - dl);
+    }
+    // dQ^T += K^T dS^T, k-step r: keys 4 j4 + r
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int i = 0; i < DU; ++i)
+        acc_dq[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+            *reinterpret_cast<const float*>(kbuf + (tb[r] ^ (i << 6))), ds[r], acc_dq[i], 0, 0, 0);
+    // the tile's reads are done: the buffers take this wave's next one
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    skip(4);
+    if (wk.valid) {
+      fetch(wk.br.k, rsk, ko, kbuf);
+      fetch(wk.br.v, rsv, vo, vbuf);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  }
+
+  // acc_dq[i][r]: dim 16 i + 4 j4 + r of query l16; a wave's sums into its own buffers
+  constexpr int PITCH = D + 4;
+  static_assert(16 * PITCH * 4 <= 2 * FT::BYTES, "a wave's sums fit its tile buffers");
+  float* const mine = reinterpret_cast<float*>(smem[w]);
+#pragma unroll
+  for (int i = 0; i < DU; ++i)
+    *reinterpret_cast<float4*>(mine + l16 * PITCH + 16 * i + 4 * j4) =
+        make_float4(acc_dq[i][0], acc_dq[i][1], acc_dq[i][2], acc_dq[i][3]);
+  __syncthreads();
+  for (int c = tid; c < 16 * (D / 4); c += 256) {
+    const int row = c / (D / 4), d = 4 * (c % (D / 4));
+    if (m0 + row >= m_end) continue;
+    float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const float4 y = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(smem[k]) +
+                                                        row * PITCH + d);
+      x.x += y.x; x.y += y.y; x.z += y.z; x.w += y.w;
+    }
+    *reinterpret_cast<float4*>(dq.at(b, m0 + row, h, d)) =
+        make_float4(x.x * scale, x.y * scale, x.z * scale, x.w * scale);
+  }
+}
+
+// dK / dV of NW x 16 keys of one block: wave w owns keys 16 w .. 16 w + 15 (K and V in registers),
+// the queries of the bucket's groups stream through LDS 16 rows at a time (two buffers).
+template <int D, int NW>
+__global__ __launch_bounds__(NW * kWave, 2) void sel_bwd_dkv_f32_kernel(
+    View4<const float> q, View4<const float> dout, DenseGrad<float> kg,
+    const float* __restrict__ nl2, const float* __restrict__ delta,
+    const int32_t* __restrict__ offsets, const int32_t* __restrict__ groups, int M, int H, int G,
+    int MG, int T, int NS, int nkt, int chunk, bool causal, float scale, int nparts) {
+  using FT = F32Tile<D>;
+  constexpr int DU = FT::DU, KT = 16 * NW;
+  constexpr int NIW = 2 * FT::NI / NW;  // this wave's copy instructions of a Q and dO tile pair
+  static_assert(NIW % 2 == 0, "whole copies of 2 or 4 instructions");
+  __shared__ __align__(16) char smem[2][2][FT::BYTES];  // [buffer][Q, dO]
+  __shared__ float rowv[2][2][64];                      // [buffer][-lse log2 e, delta]
+  const int lane = lane_id();
+  const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
+  const int l16 = lane & 15, j4 = lane >> 4;
+  const int bid = static_cast<int>(blockIdx.x) % NS;  // blocks ascending: the often selected first
+  int u0 = static_cast<int>(blockIdx.x) / NS;
+  const int kt = u0 % nkt; u0 /= nkt;
+  const int h = u0 % H;
+  const int b = u0 / H;
+  KvTile<float, float> tl;
+  if (!kg.template tile<KT>(b, h, bid, kt, tl)) return;
+  const int nk = tl.nk, t0 = tl.t0;
+  float4 kb[DU], vb[DU];
+  {
+    const int key = 16 * w + l16;
+#pragma unroll
+    for (int u = 0; u < DU; ++u) {
+      kb[u] = vb[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (key < nk) {
+        kb[u] = *reinterpret_cast<const float4*>(tl.k + key * tl.k_sn + 16 * u + 4 * j4);
+        vb[u] = *reinterpret_cast<const float4*>(tl.v + key * tl.v_sn + 16 * u + 4 * j4);
+      }
+    }
+  }
+  const float c2 = scale * kLog2e;
+  const int rb = FT::rb();
+  int tb[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) tb[r] = FT::tb(r);
+  // this wave's copies: waves of the lower half Q, of the upper half dO, NIW instructions each
+  const bool isq = w < NW / 2;
+  const int part = isq ? w : w - NW / 2;
+  const int rs = static_cast<int>(isq ? q.s1 : dout.s1) * 4;
+  int off[NIW];
+#pragma unroll
+  for (int j = 0; j < NIW; ++j) off[j] = FT::src(part * NIW + j, rs);
+  f32x4 acc_dk[DU], acc_dv[DU];
+#pragma unroll
+  for (int i = 0; i < DU; ++i) acc_dk[i] = acc_dv[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  const int64_t orow = (static_cast<int64_t>(b) * H + h) * (NS + 1);
+  const int e0 = offsets[orow + bid], e1 = offsets[orow + bid + 1];
+  const int32_t* grp = groups + (static_cast<int64_t>(b) * H + h) * (static_cast<int64_t>(MG) * T);
+  const int nitems = (e1 - e0) * nparts;
+  const int64_t lrow = (static_cast<int64_t>(b) * H + h) * M;
+  struct Item {
+    int i, q0, nq, nv;
+  };
+  int gwin = -64, gv = 0;  // bucket entries, 64 at a time, one per lane
+  auto group_of = [&](int e) -> int {
+    if ((e & ~63) != gwin) {
+      gwin = e & ~63;
+      gv = gwin + lane < e1 - e0 ? grp[e0 + gwin + lane] : 0;
+    }
+    return __builtin_amdgcn_readlane(gv, e & 63);
+  };
+  auto find = [&](int i) -> Item {  // the next 16-query part with work at or after i
+    for (; i < nitems; ++i) {
+      const int e = i / nparts, g = group_of(e);
+      const int q0 = g * G + 16 * (i - e * nparts);
+      const int nq = min(min(g * G + G, M) - q0, 16);
+      int nv = nk;
+      if (causal) {
+        const int64_t lim = static_cast<int64_t>((g * G) / chunk + 1) * chunk - t0;
+        nv = lim < nv ? static_cast<int>(lim > 0 ? lim : 0) : nv;
+      }
+      if (nq > 0 && nv > 0) return Item{i, q0, nq, nv};
+    }
+    return Item{nitems, 0, 0, 0};
+  };
+  auto issue = [&](const Item& it, int buf) {
+    const void* base = isq ? q.at(b, it.q0, h, 0) : dout.at(b, it.q0, h, 0);
+    char* dst = smem[buf][isq ? 0 : 1];
+    if constexpr (NIW == 8) {
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        const int o4[4] = {off[4 * p], off[4 * p + 1], off[4 * p + 2], off[4 * p + 3]};
+        dma_part<4>(base, rs, it.nq, dst, 2 * part + p, o4);
+      }
+    } else {
+      dma_part<NIW>(base, rs, it.nq, dst, part, off);
+    }
+    if (w < 2)
+      dma_f32x64((w == 0 ? nl2 : delta) + lrow + it.q0, lane < it.nq ? 4 * lane : -1,
+                 rowv[buf][w]);
+  };
+
+  Item cur = find(0);
+  if (cur.i < nitems) issue(cur, 0);
+  __builtin_amdgcn_s_waitcnt(0);
+  int BI = 0;
+  while (cur.i < nitems) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    const Item nx = find(cur.i + 1);
+    if (nx.i < nitems) issue(nx, BI ^ 1);
+    const char* Qt = smem[BI][0];
+    const char* Dt = smem[BI][1];
+    if (16 * w < cur.nv) {  // wave-uniform
+      // S = Q K^T and dP = dO V^T: lane holds queries 4 j4 + r of key 16 w + l16
+      f32x4 s4 = f32x4{0.f, 0.f, 0.f, 0.f}, p4 = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int u = 0; u < DU; ++u)
+        s4 = mfma4(*reinterpret_cast<const float4*>(Qt + (rb ^ (u << 6))), kb[u], s4);
+#pragma unroll
+      for (int u = 0; u < DU; ++u)
+        p4 = mfma4(*reinterpret_cast<const float4*>(Dt + (rb ^ (u << 6))), vb[u], p4);
+      const float4 L4 = *reinterpret_cast<const float4*>(rowv[BI][0] + 4 * j4);
+      const float4 D4 = *reinterpret_cast<const float4*>(rowv[BI][1] + 4 * j4);
+      const float Lr[4] = {L4.x, L4.y, L4.z, L4.w}, Dr[4] = {D4.x, D4.y, D4.z, D4.w};
+      const bool kv = 16 * w + l16 < cur.nv;
+      float pv[4], ds[4];
+      // rows past the item's queries have zero Q / dO and lse = delta = 0, so they add nothing
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        pv[r] = kv ? __builtin_amdgcn_exp2f(__builtin_fmaf(s4[r], c2, Lr[r])) : 0.0f;
+        ds[r] = pv[r] * (p4[r] - Dr[r]);
+      }
+      // dV += P^T dO and dK += dS^T Q, k-step r: queries 4 j4 + r
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int i = 0; i < DU; ++i) {
+          const int to = tb[r] ^ (i << 6);
+          acc_dv[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+              pv[r], *reinterpret_cast<const float*>(Dt + to), acc_dv[i], 0, 0, 0);
+          acc_dk[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+              ds[r], *reinterpret_cast<const float*>(Qt + to), acc_dk[i], 0, 0, 0);
+        }
+    }
+    cur = nx;
+    BI ^= 1;
+  }
+
+  // keys 16 w + 4 j4 + r, dims 16 i + l16: 64-byte runs
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int key = 16 * w + 4 * j4 + r;
+    if (key >= nk) continue;
+#pragma unroll
+    for (int i = 0; i < DU; ++i) {
+      tl.dk[key * tl.dk_sn + 16 * i + l16] = acc_dk[i][r] * scale;
+      tl.dv[key * tl.dv_sn + 16 * i + l16] = acc_dv[i][r];
+    }
+  }
+}
+
 // ---- VALU kernels (fp32 arithmetic; any element type, head dim <= 256 and strides) ------------
 // The reference's FP32 SIMT kernels (selection_bwd.cu:18-306) in the same roles: dQ walks a
 // group's blocks with 4 lanes per query (DQ dims each, dot products reduced over the 4 lanes),
@@ -1267,11 +1610,12 @@ inline BwdWs bwd_ws(int64_t B, int64_t M, int64_t H, int64_t MG, int64_t T, int6
 
 inline bool aligned16b(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-// 16-byte rows with unit dim stride, element strides in multiples of 8, rows of at least D
-// elements and 64 rows within the 32-bit tile offsets of the LDS copies.
-inline bool rows16(const omm_view4& x, int64_t D) {
-  return x.stride[3] == 1 && aligned16b(x.data) && x.stride[0] % 8 == 0 && x.stride[1] % 8 == 0 &&
-         x.stride[2] % 8 == 0 && x.stride[1] >= D && 2 * x.stride[1] * 64 < (int64_t{1} << 31);
+// 16-byte rows of es-byte elements with unit dim stride, rows of at least D elements and 64 rows
+// within the 32-bit tile offsets of the LDS copies.
+inline bool rows16(const omm_view4& x, int64_t D, int es = 2) {
+  const int64_t v = 16 / es;
+  return x.stride[3] == 1 && aligned16b(x.data) && x.stride[0] % v == 0 && x.stride[1] % v == 0 &&
+         x.stride[2] % v == 0 && x.stride[1] >= D && es * x.stride[1] * 64 < (int64_t{1} << 31);
 }
 
 // The dK / dV kernel for a call's block and group size (DM = 64 or 128): 2 waves for blocks of at
@@ -1338,12 +1682,18 @@ int sel_bwd_launch(const BwdArgs& a, char* ws, const BwdWs& L, hipStream_t s) {
   DenseAcc<QT> acc{make_view<const QT>(k), make_view<const QT>(v),
                    static_cast<const int32_t*>(ids.data), ids.stride[0], ids.stride[1],
                    ids.stride[2], ids.stride[3], N, bs, ch, causal};
-  const int64_t dq_items = static_cast<int64_t>(B) * H * MG * nsub;
-  const int nkt = (bs + 63) / 64;
+  constexpr bool F32 = DM > 0 && sizeof(QT) == 4;  // the fp32 MFMA kernels
+  const int nsub16 = (G + 15) / 16;
+  const int64_t dq_items = static_cast<int64_t>(B) * H * MG * (F32 ? nsub16 : nsub);
+  const int nkt = F32 && bs <= 32 ? 1 : (bs + 63) / 64;
   const int64_t kv_items = static_cast<int64_t>(B) * H * NS * nkt;
   OMM_REQUIRE(dq_items <= 2147483647ll && kv_items <= 2147483647ll, OMM_EUNSUPPORTED,
               "omm_sel_bwd: grid too large");
-  if constexpr (DM > 0) {
+  if constexpr (F32) {
+    sel_bwd_dq_f32_kernel<DenseAcc<QT>, DM><<<static_cast<unsigned>(dq_items), 256, 0, s>>>(
+        make_view<const QT>(q), make_view<const QT>(*a.out), make_view<const QT>(*a.dout),
+        make_view<QT>(*a.dq), a.lse, delta, nl2, acc, M, H, G, MG, T, ch, a.scale, nsub16);
+  } else if constexpr (DM > 0) {
     launch_dq<QT, DenseAcc<QT>, DM>(q, *a.out, *a.dout, *a.dq, a.lse, delta, nl2, acc, M, H, G, MG,
                                     T, ch, a.scale, nsub, dq_items, s);
   } else {
@@ -1366,7 +1716,16 @@ int sel_bwd_launch(const BwdArgs& a, char* ws, const BwdWs& L, hipStream_t s) {
   if (kv_items == 0) return OMM_OK;
   const DenseGrad<QT> kg{make_view<const QT>(k), make_view<const QT>(v), make_view<QT>(*a.dk),
                          make_view<QT>(*a.dv), N, bs};
-  if constexpr (DM > 0) {
+  if constexpr (F32) {
+    auto run = [&](auto nw) {
+      constexpr int NW = decltype(nw)::value;
+      sel_bwd_dkv_f32_kernel<DM, NW><<<static_cast<unsigned>(kv_items), NW * kWave, 0, s>>>(
+          make_view<const QT>(q), make_view<const QT>(*a.dout), kg, nl2, delta, offsets, groups, M,
+          H, G, MG, T, NS, nkt, ch, causal, a.scale, nsub16);
+    };
+    if (bs <= 32) run(std::integral_constant<int, 2>{});
+    else run(std::integral_constant<int, 4>{});
+  } else if constexpr (DM > 0) {
     return launch_dkv<QT, DM>(q, *a.dout, kg, nl2, delta, offsets, groups, M, H, G, MG, T, NS, bs,
                               ch, causal, a.scale, s);
   } else {
@@ -1444,6 +1803,9 @@ int sel_bwd_typed(const BwdArgs& a, bool mfma, char* ws, const BwdWs& L, hipStre
   if constexpr (sizeof(QT) == 2) {
     if (mfma && D == 128) return sel_bwd_launch<QT, 128, 0>(a, ws, L, s);
     if (mfma && D == 64) return sel_bwd_launch<QT, 64, 0>(a, ws, L, s);
+  } else {
+    if (mfma && D == 128) return sel_bwd_launch<QT, 128, 0>(a, ws, L, s);
+    if (mfma && D == 64) return sel_bwd_launch<QT, 64, 0>(a, ws, L, s);
   }
   if (D <= 64) return sel_bwd_launch<QT, 0, 16>(a, ws, L, s);
   if (D <= 128) return sel_bwd_launch<QT, 0, 32>(a, ws, L, s);
@@ -1499,11 +1861,13 @@ extern "C" int omm_sel_bwd(const omm_view4* q, const omm_view4* k, const omm_vie
   OMM_REQUIRE(D >= 1 && D <= 256, OMM_EUNSUPPORTED, "omm_sel_bwd: head dim must be in [1, 256] "
               "(got %lld)", (long long)D);
   OMM_REQUIRE(__builtin_isfinite(scale), OMM_EINVAL, "omm_sel_bwd: scale must be finite");
-  // MFMA kernels: 16-bit rows of head dim 64 / 128, 16-byte aligned, and a non-zero scale;
-  // everything else runs the VALU kernels (k and v then need one dim stride)
+  // MFMA kernels: rows of head dim 64 / 128, 16-byte aligned, and a non-zero scale; everything
+  // else runs the VALU kernels (k and v then need one dim stride)
   bool rows_ok = true;
-  for (const omm_view4* x : {q, k, v, out, dout, dq, dk, dv}) rows_ok = rows_ok && rows16(*x, D);
-  const bool mfma = (dtype == OMM_BF16 || dtype == OMM_F16) && (D == 64 || D == 128) && rows_ok &&
+  const int es = dtype == OMM_F32 ? 4 : 2;
+  for (const omm_view4* x : {q, k, v, out, dout, dq, dk, dv})
+    rows_ok = rows_ok && rows16(*x, D, es);
+  const bool mfma = (D == 64 || D == 128) && rows_ok &&
                     scale != 0.0f && M < (int64_t{1} << 29);
   OMM_REQUIRE(mfma || k->stride[3] == v->stride[3], OMM_EUNSUPPORTED,
               "omm_sel_bwd: k and v need the same dim stride");
@@ -1514,7 +1878,7 @@ extern "C" int omm_sel_bwd(const omm_view4* q, const omm_view4* k, const omm_vie
   switch (dtype) {
     case OMM_BF16: return sel_bwd_typed<bf16_t>(a, mfma, ws, L, s);
     case OMM_F16: return sel_bwd_typed<f16_t>(a, mfma, ws, L, s);
-    case OMM_F32: return sel_bwd_typed<float>(a, false, ws, L, s);
+    case OMM_F32: return sel_bwd_typed<float>(a, mfma, ws, L, s);
     default: return set_error(OMM_EINVAL, "omm_sel_bwd: unsupported dtype %d", dtype);
   }
 }

@@ -127,6 +127,28 @@ def test_sel_bwd_block_and_group_edges(BS, G, D):
         _close(name, got, w)
 
 
+@pytest.mark.parametrize("BS", [15, 16, 32, 33, 64, 65])
+@pytest.mark.parametrize("G", [1, 15, 16, 17, 33, 64])
+@pytest.mark.parametrize("D", [64, 128])
+def test_sel_bwd_f32_block_and_group_edges(BS, G, D):
+    """The fp32 MFMA kernels around their 16-query and 16-key tiles: groups and blocks that fill,
+    split and do not fill them, fewer key tiles than waves, a ragged last group and block, -1 ids,
+    chunk-causal prefixes that cut blocks and a negative scale."""
+    M, N, H, T, chunk = 100, 210, 2, 3, 90
+    gen = torch.Generator().manual_seed(BS * 100 + G)
+    q, k, v = (torch.randn((1, L, H, D), generator=gen) for L in (M, N, N))
+    ids = _ids(gen, 1, -(-M // G), H, T, -(-N // BS), 0.1)
+    scale = -D ** -0.5 if BS == 33 else D ** -0.5
+    out, lse, do, dq, dk, dv, _ = _run(q, k, v, ids, G, BS, True, chunk, torch.float32, scale)
+    want = O.selection_attention_bwd(q.double().numpy(), k.double().numpy(), v.double().numpy(),
+                                     ids.numpy(), out.double().cpu().numpy(),
+                                     lse.double().cpu().numpy(), do.double().numpy(), G, scale,
+                                     O.dense_block_tokens(N, BS, chunk, True), chunk_size=chunk,
+                                     causal=True)
+    for name, got, w in (("dq", dq, want[0]), ("dk", dk, want[1]), ("dv", dv, want[2])):
+        _close(name, got, w, *TOL[torch.float32])
+
+
 # fp32 everywhere; bf16 only at head dims the MFMA kernels do not take (bf16 at 64 / 128 runs
 # the MFMA kernels, covered by test_sel_bwd_matches_oracle)
 VALU_PARAMS = [pytest.param(case, dt, id=f"valu{i}-{'f32' if dt == torch.float32 else 'bf16'}")
