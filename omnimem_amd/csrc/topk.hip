@@ -22,6 +22,8 @@
 //      Column chunk ids are precomputed once per workgroup in LDS.
 //   Rows whose columns are split over several workgroups (long key histories) write packed
 //   keys and a merge kernel selects again over the per-span winners.
+// bf16 / f16 rows on MFMA: topk <= 16 takes its scores from there, topk 17..64 only a pre-selection
+// ahead of the fmaf-chain scores (the sections below).
 // topk > 128 (the reference's path B): the same scoring writes every row's scores to the
 // workspace and topk_large_kernel selects per row (radix select, then an LDS bitonic sort).
 #include "omm_common.h"
@@ -1639,6 +1641,296 @@ __global__ __launch_bounds__(kM2Threads, 2) void topk_mfma_kernel(M2Args a) {
   }
 }
 
+// ---- MFMA pre-selection with exact scores (16 < topk <= 64) --------------------------------------
+// The same inputs as above, but the indices are those of the fmaf-chain scores (topk_kernel's), bit
+// for bit.  MFMA scores s' pick the candidates: both sums differ from the exact dot product by at
+// most D 2^-24 sum |q_d k_d| <= D 2^-24 |q| |k|, so with E = 4 D 2^-24 |q| max |k| |scale| (twice the
+// two bounds; it also covers the rounding of the product with scale) every column of the exact top
+// topk has s' >= x - 2 E for any x that at least topk columns reach.  x comes from bisecting the
+// row's range of s' until it leaves topk to topk + 40 columns; the candidates (about as many:
+// random scores leave a tenth of a column within 2 E) are scored by the fmaf chain, one lane each,
+// and ranked.  A row whose norms are not between 1e-15 and 1e15 (the bound needs products and sums
+// clear of overflow and of the denormal range), whose ties leave more than kExCand candidates or
+// whose bisection does not end scores every visible column by the chain instead.
+// Bound by the latencies of the phases between the barriers (column loads, bisection, candidate
+// gathers) at one workgroup per CU, so one row per wave and 16 waves.  Against topk_kernel, whose
+// fp32 vector scoring and selection of every column take most of its time, with the pooling: top-64
+// of 1365 columns, 16380 rows: 295 -> 137 us (top-20: 241 -> 111); top-32 of 512 columns, 6144 rows:
+// 59 -> 48 us; top-64 of 5920 columns in spans, 888 rows: 118 -> 79 us.
+constexpr int kExWaves = 16;
+constexpr int kExThreads = kExWaves * kWave;
+constexpr int kExSpanCap = 1792;  // columns per item: 28 a lane, 115 KiB of scores
+constexpr int kExCand = 128;      // candidates per row, two a lane
+constexpr int kExMaxTopk = 64;
+constexpr float kExNorm2Min = 1e-30f, kExNorm2Max = 1e30f;
+
+__host__ __device__ inline int ex_pitch(int span) { return span + 4; }  // span: a multiple of 16
+inline size_t ex_lds_bytes(int span, int D) {
+  return static_cast<size_t>(kM2Rows) * ex_pitch(span) * 4 + static_cast<size_t>(kM2Rows) * D * 4 +
+         static_cast<size_t>(kM2Rows) * (D + 8) * 2 + static_cast<size_t>(kExWaves) * kSurvCap * 8;
+}
+
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// JM: 64-column steps a lane holds (span <= 64 JM)
+template <typename T, int D, int JM>
+__global__ __launch_bounds__(kExThreads) void topk_exact_kernel(M2Args a) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  constexpr int SD = D / 32, CH = D / 8, QP = D + 8;
+  __shared__ RowCols facts[kM2Rows];
+  __shared__ float qn2[kM2Rows];
+  __shared__ uint32_t kn2;  // bits of the largest |k|^2 (non-negative floats order as integers)
+  __shared__ int kbad;      // some |k|^2 is not finite
+  const int tid = threadIdx.x, lane = lane_id();
+  const int w = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int l16 = lane & 15, j4 = lane >> 4;
+  int it = xcd_remap(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x));
+  const int rt = a.rtiles - 1 - it % a.rtiles; it /= a.rtiles;
+  const int sp = it % a.nspan; it /= a.nspan;
+  const int h = it % a.H;
+  const int b = it / a.H;
+  const int row0 = rt * kM2Rows, SP = ex_pitch(a.span), c_begin = sp * a.span;
+  float* sc = reinterpret_cast<float*>(smem);
+  float* qf = reinterpret_cast<float*>(smem + a.o_qs) - kM2Rows * D;  // the rows in fp32
+  uint16_t* qs = reinterpret_cast<uint16_t*>(smem + a.o_qs);
+  uint64_t* sv = reinterpret_cast<uint64_t*>(smem + a.o_sv) + w * kSurvCap;
+  const T* qp = static_cast<const T*>(a.q) + b * a.qs0 + h * a.qs2;
+  const T* kp = static_cast<const T*>(a.k) + b * a.ks0 + h * a.ks2;
+
+  // ---- 1. row facts, rows and their norms ----
+  int ub;
+  {
+    const int g = row0 + l16;
+    RowCols rc{0, 0, 0, 0};
+    if (g < a.MG) rc = row_cols(a.mk, row_info(a.mk, g), a.NC);
+    if (w == 0 && lane < kM2Rows) facts[lane] = rc;
+    ub = static_cast<int>(row16_max(static_cast<uint32_t>(max(rc.hi0, rc.hi1))));
+    ub = __builtin_amdgcn_readfirstlane(ub);
+  }
+  const int n = max(0, min(c_begin + a.span, ub) - c_begin), nblk = (n + 15) / 16;
+  if (tid == 0) {
+    kn2 = 0u;
+    kbad = 0;
+  }
+  if (tid < kM2Rows * CH) {
+    const int pr = tid / CH, pu = tid - pr * CH;
+    uint4 val = make_uint4(0, 0, 0, 0);
+    if (row0 + pr < a.MG)
+      val = *reinterpret_cast<const uint4*>(qp + static_cast<int64_t>(row0 + pr) * a.qs1 + pu * 8);
+    *reinterpret_cast<uint4*>(qs + pr * QP + pu * 8) = val;
+    float f[8], ss = 0.0f;
+    unpack<T>(val, f);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      qf[pr * D + pu * 8 + i] = f[i];
+      ss = __builtin_fmaf(f[i], f[i], ss);
+    }
+#pragma unroll
+    for (int m = 1; m < CH; m <<= 1) ss += __shfl_xor(ss, m, kWave);
+    if (pu == 0) qn2[pr] = ss;
+  }
+  __syncthreads();
+
+  // ---- 2. S^T = K Qp^T on MFMA -> LDS, and the columns' largest norm: of the products of a block's
+  // columns with each other the largest is a column's own square ----
+  {
+    uint4 qb[SD];
+#pragma unroll
+    for (int s = 0; s < SD; ++s)
+      qb[s] = *reinterpret_cast<const uint4*>(qs + l16 * QP + 32 * s + 8 * j4);
+    float kmax = 0.0f;
+    bool bad = false;
+    for (int cb = w; cb < nblk; cb += kExWaves) {
+      const int col = min(c_begin + cb * 16 + l16, a.NC - 1);
+      uint4 kf[SD];
+#pragma unroll
+      for (int s = 0; s < SD; ++s)
+        kf[s] = *reinterpret_cast<const uint4*>(kp + static_cast<int64_t>(col) * a.ks1 + 32 * s + 8 * j4);
+      m2_f32x4 acc = m2_f32x4{0.f, 0.f, 0.f, 0.f}, kk = acc;
+#pragma unroll
+      for (int s = 0; s < SD; ++s) {
+        acc = M2Mfma<T>::run(kf[s], qb[s], acc);
+        kk = M2Mfma<T>::run(kf[s], kf[s], kk);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        bad = bad || !(kk[i] <= kExNorm2Max);
+        kmax = fmaxf(kmax, kk[i]);
+      }
+      *reinterpret_cast<float4*>(sc + l16 * SP + cb * 16 + 4 * j4) =
+          make_float4(acc[0] * a.scale, acc[1] * a.scale, acc[2] * a.scale, acc[3] * a.scale);
+    }
+    const uint32_t km = wave_max_u32(__builtin_bit_cast(uint32_t, kmax));
+    if (lane == 0) atomicMax(&kn2, km);
+    if (bad) kbad = 1;
+  }
+  __syncthreads();
+
+  // ---- 3. one row per wave ----
+  const int r = w, g = row0 + r, NC = a.NC, topk = a.topk;
+  if (g >= a.MG) return;  // wave-uniform; no workgroup barrier below
+  const RowCols rc = clip_cols(facts[r], c_begin, n);
+  const int64_t orow = (static_cast<int64_t>(b) * a.MG + g) * a.H + h;
+  float* srow = sc + r * SP;
+  auto emit = [&](int rank, uint64_t kk) {
+    if (a.nspan == 1) a.out[orow * topk + rank] = key_id(kk, NC);
+    else a.part[(orow * a.nspan + sp) * topk + rank] = kk;
+  };
+  auto pad = [&](int p) {
+    if (a.nspan == 1) a.out[orow * topk + p] = -1;
+    else a.part[(orow * a.nspan + sp) * topk + p] = 0ull;
+  };
+  // topk_kernel's score of NS columns: fmaf over d ascending from 0, then * scale
+  auto chain = [&](auto ns, const int* col, float* res) {
+    constexpr int NS = decltype(ns)::value;
+    const T* kr[NS];
+    float acc[NS];
+#pragma unroll
+    for (int m = 0; m < NS; ++m) {
+      kr[m] = kp + static_cast<int64_t>(c_begin + col[m]) * a.ks1;
+      acc[m] = 0.0f;
+    }
+#pragma unroll
+    for (int d0 = 0; d0 < D; d0 += 32) {
+      uint4 kv[NS][4];
+#pragma unroll
+      for (int m = 0; m < NS; ++m)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) kv[m][u] = *reinterpret_cast<const uint4*>(kr[m] + d0 + 8 * u);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        float4 q4[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+          q4[e] = *reinterpret_cast<const float4*>(qf + r * D + d0 + 8 * u + 4 * e);
+#pragma unroll
+        for (int m = 0; m < NS; ++m) {
+          float f[8];
+          unpack<T>(kv[m][u], f);
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            acc[m] = __builtin_fmaf(q4[e].x, f[4 * e], acc[m]);
+            acc[m] = __builtin_fmaf(q4[e].y, f[4 * e + 1], acc[m]);
+            acc[m] = __builtin_fmaf(q4[e].z, f[4 * e + 2], acc[m]);
+            acc[m] = __builtin_fmaf(q4[e].w, f[4 * e + 3], acc[m]);
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int m = 0; m < NS; ++m) res[m] = acc[m] * a.scale;
+  };
+
+  const int nvis = (rc.hi0 - rc.lo0) + (rc.hi1 - rc.lo1);
+  const float q2 = qn2[r], k2 = __builtin_bit_cast(float, kn2);
+  const float E = 4.0f * D * 0x1p-24f * __builtin_sqrtf(q2) * __builtin_sqrtf(k2) * fabsf(a.scale);
+  bool ok = kbad == 0 && q2 >= kExNorm2Min && q2 <= kExNorm2Max && k2 >= kExNorm2Min &&
+            fabsf(a.scale) >= 1e-6f && fabsf(a.scale) <= 1e10f;
+  uint16_t* const list = reinterpret_cast<uint16_t*>(sv + kExCand);  // behind the candidates' keys
+  int nc = 0;
+  if (ok && nvis > 0) {
+    // (steps past the tile's last column are skipped four at a time: a causal tile has fewer)
+    float v[JM];
+    float vmax = kNegInf, vmin = -kNegInf;
+    const bool one = rc.lo1 >= rc.hi1;  // wave-uniform: one run of columns
+#pragma unroll
+    for (int j0 = 0; j0 < JM; j0 += 4) {
+      if (64 * j0 < n) {
+#pragma unroll
+        for (int j = j0; j < j0 + 4; ++j) {
+          const int i = 64 * j + lane;
+          const float x = srow[min(i, n - 1)];
+          const bool in = one ? i >= rc.lo0 && i < rc.hi0 : in_cols(rc, i);
+          v[j] = in ? x : kNegInf;
+          vmax = fmaxf(vmax, v[j]);
+          vmin = fminf(vmin, in ? x : -kNegInf);
+        }
+      }
+    }
+    float thr = kNegInf;  // every visible column, unless they are more than the candidate slots
+    if (nvis > kExCand) {
+      vmax = wave_max_xor(vmax, 1, 32);
+      float lo = -wave_max_xor(-vmin, 1, 32), hi = vmax;  // at least topk columns reach lo
+      bool found = false;
+      for (int round = 0; round < 24 && !found; ++round) {
+        const float mid = 0.5f * (lo + hi);
+        int c = 0;
+#pragma unroll
+        for (int j0 = 0; j0 < JM; j0 += 4) {
+          if (64 * j0 < n) {
+#pragma unroll
+            for (int j = j0; j < j0 + 4; ++j) c += popc64(ballot64(v[j] >= mid));
+          }
+        }
+        if (c >= topk) lo = mid;
+        else hi = mid;
+        found = c >= topk && c <= topk + 40;
+      }
+      ok = found;
+      thr = lo - 2.0f * E;
+    }
+    if (ok) {
+#pragma unroll
+      for (int j0 = 0; j0 < JM; j0 += 4) {
+        if (64 * j0 < n) {
+#pragma unroll
+          for (int j = j0; j < j0 + 4; ++j) {
+            // (v is -inf for a hidden column; a visible one is finite here)
+            const bool surv = v[j] >= thr && v[j] > kNegInf;
+            const uint64_t m = ballot64(surv);
+            const int pos = nc + lanes_below(m);
+            if (surv && pos < kExCand) list[pos] = static_cast<uint16_t>(64 * j + lane);
+            nc += popc64(m);
+          }
+        }
+      }
+      ok = nc <= kExCand;
+    }
+  }
+  if (!ok) {  // wave-uniform: every visible column by the chain, then the general selection
+    for (int i = lane; i < n; i += kWave)
+      if (in_cols(rc, i)) chain(std::integral_constant<int, 1>{}, &i, &srow[i]);
+    wave_lds_fence();
+    wave_select(n, topk,
+                [&](int i) -> uint64_t { return in_cols(rc, i) ? make_key(srow[i], c_begin + i, NC) : 0ull; },
+                emit, pad, sv);
+    return;
+  }
+  wave_lds_fence();
+  uint64_t mine[2];
+  int col[2];
+  float x[2] = {0.0f, 0.0f};
+#pragma unroll
+  for (int m = 0; m < 2; ++m) col[m] = lane + kWave * m < nc ? list[lane + kWave * m] : 0;
+  if (nc > kWave) chain(std::integral_constant<int, 2>{}, col, x);
+  else chain(std::integral_constant<int, 1>{}, col, x);
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    const int i = lane + kWave * m;
+    mine[m] = i < nc ? make_key(x[m], c_begin + col[m], NC) : 0ull;
+    sv[i] = mine[m];
+  }
+  wave_lds_fence();
+  int rank[2] = {0, 0};
+  for (int j = 0; j < nc; j += 8) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const ulonglong2 y = reinterpret_cast<const ulonglong2*>(sv + j)[e];
+#pragma unroll
+      for (int m = 0; m < 2; ++m) rank[m] += (y.x > mine[m] ? 1 : 0) + (y.y > mine[m] ? 1 : 0);
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < 2; ++m)
+    if (mine[m] != 0ull && rank[m] < topk) emit(rank[m], mine[m]);
+  for (int p = lane; p < topk; p += kWave)
+    if (p >= nc) pad(p);
+}
+
 // ---- host planning ---------------------------------------------------------------------------
 int span_cap(int D, int esize, bool scores) {
   for (int s = kSpanCap; s > kTileC; s -= kTileC)
@@ -1820,6 +2112,13 @@ bool m2_ok(int32_t dtype, const omm_view4& q, const omm_view4& k, int topk) {
   return (D == 64 || D == 128) && m2_view_ok(q) && m2_view_ok(k);
 }
 
+// the same inputs with 16 < topk <= 64: exact scores behind an MFMA pre-selection
+bool ex_ok(int32_t dtype, const omm_view4& q, const omm_view4& k, int topk) {
+  if (dtype != OMM_BF16 && dtype != OMM_F16) return false;
+  const int64_t D = q.size[3];
+  return topk > 16 && topk <= kExMaxTopk && (D == 64 || D == 128) && m2_view_ok(q) && m2_view_ok(k);
+}
+
 struct M2Plan {
   int span, nspan, rtiles;
   size_t ws_part;
@@ -1839,6 +2138,21 @@ M2Plan m2_plan(int64_t B, int64_t MG, int64_t H, int64_t NC, int topk, bool fuse
   if (span < 16) span = 16;
   p.span = static_cast<int>(span);
   p.nspan = static_cast<int>(std::max<int64_t>(1, cdiv64(NC, span)));
+  p.ws_part = p.nspan > 1 ? static_cast<size_t>(B * MG * H) * p.nspan * topk * sizeof(uint64_t) : 0;
+  return p;
+}
+
+// One item covers a row tile's columns when they fit its LDS; else, or with few row tiles, they are
+// split so that about 512 items run, and the merge kernel selects again over the spans' winners.
+M2Plan ex_plan(int64_t B, int64_t MG, int64_t H, int64_t NC, int topk) {
+  M2Plan p{};
+  p.rtiles = static_cast<int>(cdiv64(MG, kM2Rows));
+  const int64_t tiles = B * H * p.rtiles;
+  int64_t nspan = cdiv64(NC, kExSpanCap);
+  if (tiles * nspan < 512)
+    nspan = std::max(nspan, std::min(cdiv64(512, tiles), cdiv64(NC, 512)));
+  p.span = static_cast<int>((cdiv64(NC, nspan) + 15) / 16 * 16);
+  p.nspan = static_cast<int>(std::max<int64_t>(1, cdiv64(NC, p.span)));
   p.ws_part = p.nspan > 1 ? static_cast<size_t>(B * MG * H) * p.nspan * topk * sizeof(uint64_t) : 0;
   return p;
 }
@@ -1871,6 +2185,48 @@ int launch_m2_typed(M2Args a, int64_t B, int64_t H, const M2Plan& p, hipStream_t
   topk_merge_kernel<<<static_cast<unsigned>(cdiv64(rows, kWaves)), kThreads, 0, s>>>(
       a.part, a.out, rows, p.nspan, a.topk, a.NC);
   return check_launch("top-k merge");
+}
+
+template <typename T, int D>
+int launch_ex_typed(M2Args a, int64_t B, int64_t H, const M2Plan& p, hipStream_t s) {
+  const size_t lds = ex_lds_bytes(p.span, D);
+  a.span = p.span;
+  a.nspan = p.nspan;
+  a.rtiles = p.rtiles;
+  a.o_qs = static_cast<uint32_t>(static_cast<size_t>(kM2Rows) * (ex_pitch(p.span) + D) * 4);
+  a.o_sv = static_cast<uint32_t>(a.o_qs + static_cast<size_t>(kM2Rows) * (D + 8) * 2);
+  const int64_t items = B * H * p.nspan * p.rtiles;
+  OMM_REQUIRE(items <= 2147483647ll, OMM_EUNSUPPORTED, "top-k: grid too large");
+  auto run = [&](auto jm) -> int {
+    constexpr int JM = decltype(jm)::value;
+    const void* f = reinterpret_cast<const void*>(&topk_exact_kernel<T, D, JM>);
+    if (lds > 64 * 1024) {
+      const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                               static_cast<int>(lds));
+      if (e != hipSuccess)
+        return set_error(OMM_EHIP, "top-k: LDS attribute: %s", hipGetErrorString(e));
+    }
+    topk_exact_kernel<T, D, JM><<<static_cast<unsigned>(items), kExThreads, lds, s>>>(a);
+    return check_launch("top-k (exact)");
+  };
+  int rc;
+  if (p.span <= 512) rc = run(std::integral_constant<int, 8>{});
+  else if (p.span <= 1024) rc = run(std::integral_constant<int, 16>{});
+  else rc = run(std::integral_constant<int, 28>{});
+  if (rc != OMM_OK || p.nspan == 1) return rc;
+  const int64_t rows = B * a.MG * H;
+  topk_merge_kernel<<<static_cast<unsigned>(cdiv64(rows, kWaves)), kThreads, 0, s>>>(
+      a.part, a.out, rows, p.nspan, a.topk, a.NC);
+  return check_launch("top-k merge");
+}
+
+int launch_ex(int32_t dtype, int D, const M2Args& a, int64_t B, int64_t H, const M2Plan& p,
+              hipStream_t s) {
+  if (dtype == OMM_BF16)
+    return D == 128 ? launch_ex_typed<bf16_t, 128>(a, B, H, p, s)
+                    : launch_ex_typed<bf16_t, 64>(a, B, H, p, s);
+  return D == 128 ? launch_ex_typed<f16_t, 128>(a, B, H, p, s)
+                  : launch_ex_typed<f16_t, 64>(a, B, H, p, s);
 }
 
 template <bool FUSED>
@@ -1947,6 +2303,15 @@ extern "C" int omm_topk(const omm_view4* q, const omm_view4* k, int32_t dtype, i
                 workspace_bytes);
     const M2Args a = m2_args(*q, *k, MG, H, NC, topk, scale, *mask, out, workspace, nullptr);
     return launch_m2<false>(dtype, static_cast<int>(D), a, B, H, p, s);
+  }
+  // (the pre-selection's spans need other scratch than the general path's: where the given one does
+  // not hold them, the general path, of the same indices, runs as it did)
+  if (ex_ok(dtype, *q, *k, topk)) {
+    const M2Plan p = ex_plan(B, MG, H, NC, topk);
+    if (p.ws_part == 0 || (workspace != nullptr && p.ws_part <= workspace_bytes)) {
+      const M2Args a = m2_args(*q, *k, MG, H, NC, topk, scale, *mask, out, workspace, nullptr);
+      return launch_ex(dtype, static_cast<int>(D), a, B, H, p, s);
+    }
   }
   if (topk > kMaxTopk) {  // scores to the workspace, then the per-row selection
     const size_t need = large_ws_bytes(B, MG, H, NC);
@@ -2071,6 +2436,25 @@ int topk_fused_impl(const omm_view4* q, const omm_view4* k, int32_t dtype, int32
     rc = launch_typed<kModePooled>(dtype, a, B, MG, H, p, static_cast<int>(D), s);
     if (rc) return rc;
     return launch_large(sc, B, MG, H, NC, topk, *mask, out, s);
+  }
+
+  if (ex_ok(dtype, *q, *k, topk)) {  // pool once into the workspace
+    const size_t pooled_bytes = align256(static_cast<size_t>(B * MG * H * D) * es);
+    const M2Plan p = ex_plan(B, MG, H, NC, topk);
+    // (a smaller or unaligned workspace, or a grid larger than the pooling's: the general path)
+    if (workspace != nullptr && pooled_bytes + p.ws_part <= workspace_bytes &&
+        (reinterpret_cast<uintptr_t>(workspace) & 15u) == 0 && MG <= 65535 && B <= 65535) {
+      omm_view4 pooled{};
+      pooled.data = workspace;
+      pooled.size[0] = B; pooled.size[1] = MG; pooled.size[2] = H; pooled.size[3] = D;
+      pooled.stride[3] = 1; pooled.stride[2] = D; pooled.stride[1] = H * D;
+      pooled.stride[0] = MG * H * D;
+      rc = pool_launch(*q, pooled, dtype, group_size, s);
+      if (rc) return rc;
+      const M2Args a = m2_args(pooled, *k, MG, H, NC, topk, scale, *mask, out,
+                               static_cast<unsigned char*>(workspace) + pooled_bytes, nullptr);
+      return launch_ex(dtype, static_cast<int>(D), a, B, H, p, s);
+    }
   }
 
   const bool vec = vec_ok(*q, es) && vec_ok(*k, es);

@@ -379,6 +379,58 @@ def test_topk_fused_massive_ties_bitexact():
     assert (got[:, :, :2] == np.arange(16)).all()  # all-zero scores: the lowest ids
 
 
+# The exact selection of 17..64 of 16-bit rows: spans of 8, 16 and 28 column steps, one span and
+# several (the merge), rows with fewer visible columns than topk, than the candidate slots and more,
+# and the rows that leave the pre-selection: ties, infinities and NaN, norms out of its range.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("data", ["random", "ties", "nonfinite", "tiny", "skewed"])
+@pytest.mark.parametrize("T,NC,H,D,G,topk,kw", [
+    (1000, 40, 2, 64, 15, 17, dict(block_size=15, chunk_size=300, causal=True)),
+    (700, 129, 3, 128, 1, 64, dict(block_size=6, chunk_size=60, causal=True)),
+    (2048, 512, 1, 128, 64, 33, dict(block_size=4, chunk_size=512, causal=True, tf_mask=True)),
+    (16380, 1365, 4, 128, 24, 64, dict(block_size=12, chunk_size=2340, causal=True)),
+    (4680, 1024, 12, 64, 9, 32, dict(block_size=64, chunk_size=4680, causal=False,
+                                     exclude_window_chunks=2, q_chunk_offset=9,
+                                     blocks_per_chunk=74, progressive_exclude=True)),
+    (2100, 1793, 24, 64, 4, 64, dict(block_size=2, chunk_size=700, causal=True)),
+    (300, 5920, 2, 128, 30, 50, dict(block_size=64, chunk_size=4680, causal=False,
+                                     exclude_window_chunks=3, q_chunk_offset=79,
+                                     blocks_per_chunk=74)),
+])
+def test_topk_exact_preselection_matches_general_path(dtype, data, T, NC, H, D, G, topk, kw):
+    from omnimem_amd.index_topk import parallel_nsa_topk
+    g = torch.Generator().manual_seed(NC + topk)
+    q = torch.randn((1, T, H, D), generator=g)
+    k = torch.randn((1, NC, H, D), generator=g)
+    if data == "ties":
+        k = torch.randint(-1, 2, k.shape, generator=g).float() / 8
+        k[:, :, 0] = 0
+        q = torch.randint(-2, 3, q.shape, generator=g).float()
+    elif data == "nonfinite":
+        k[:, ::7, 0, 3] = float("inf")
+        k[:, 1::11, 0, 5] = float("nan")
+        k[:, 2::5, 0, 7] = -float("inf")
+        q[:, : T // 2, H - 1] = 0.0  # zero rows: every score 0
+        q[:, T // 2 + 1, H - 1, 1] = float("inf")
+    elif data == "tiny":  # f16 denormals; bf16 products near the bottom of the norms' range
+        k *= 2.0 ** -22 if dtype == torch.float16 else 2.0 ** -52
+        q *= 2.0 ** -16 if dtype == torch.float16 else 2.0 ** -46
+    elif data == "skewed":  # a few columns far above the rest, the rest within rounding errors
+        k = k[:, :1] + k * 2.0 ** -9
+        k[:, ::97] *= 30.0
+    q, k = q.to(dtype).to(DEV), k.to(dtype).to(DEV)
+    odd = torch.zeros((1, NC, H, D + 1), dtype=dtype, device=DEV)[..., :D]
+    odd.copy_(k)  # rows off 16 bytes: the general path
+    got = parallel_nsa_topk(q, k, topk, group_size=G, **kw)
+    want = parallel_nsa_topk(q, odd, topk, group_size=G, **kw)
+    assert torch.equal(got, want), int((got != want).sum())
+    if NC <= 40 and data != "nonfinite":
+        name = "bf16" if dtype == torch.bfloat16 else "f16"
+        mask = O.Mask(block_size=15, group_size=G, chunk_q=300, chunk_k=300, causal=1)
+        np.testing.assert_array_equal(
+            got.cpu().numpy(), O.topk(O.pool_mean(_img(q), G, name), _img(k), topk, D ** -0.5, mask))
+
+
 # Mask modes on the MFMA path's four-rows-per-wave selection, whose visibility is a pair of
 # column intervals per row (one visible run, plus a noisy row's own noisy chunk under tf_mask or
 # the chunks past a non-causal exclusion window).  Each case is (T, NC, H, D, G, topk, facade
