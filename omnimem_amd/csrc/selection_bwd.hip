@@ -475,9 +475,27 @@ void launch_dq(const omm_view4& q, const omm_view4& out, const omm_view4& dout, 
 }
 
 // ---- block -> query-group index --------------------------------------------------------------
-constexpr int kIdxThreads = 512;
+constexpr int kIdxThreads = 1024;
 constexpr int kIdxWaves = kIdxThreads / kWave;
 constexpr int kIdxBuckets = 64;  // buckets per workgroup
+constexpr int kIdxList = 512;    // listed pairs per wave
+
+// n / d for every 32-bit n by a multiplication (Granlund and Montgomery, "Division by invariant
+// integers using multiplication", PLDI 1994, figure 4.1); d >= 1.
+struct FastDiv {
+  uint32_t m, sh1, sh2;
+  explicit FastDiv(uint32_t d) {
+    uint32_t l = 0;
+    while ((1ull << l) < d) ++l;
+    m = static_cast<uint32_t>(((1ull << 32) * ((1ull << l) - d)) / d + 1);
+    sh1 = std::min(l, 1u);
+    sh2 = l > 0 ? l - 1 : 0;
+  }
+  __device__ __forceinline__ uint32_t operator()(uint32_t n) const {
+    const uint32_t t = __umulhi(m, n);
+    return (t + ((n - t) >> sh1)) >> sh2;
+  }
+};
 
 // Bucket of (group g, slot t) of row (b, h), or -1 when the pair reaches no key.  Ids at or past
 // the row's limit (NS, or n_blocks[h] when that is smaller) reach none.
@@ -487,20 +505,27 @@ struct PairBucket {
   int T, NS, bs, chunk, G;
   bool causal;
   const int32_t* n_blocks;  // per-head bound, or nullptr
+  FastDiv by_t, by_chunk;   // T (1 if there is no pair) and chunk
+  __device__ __forceinline__ int group(int p) const {
+    return static_cast<int>(by_t(static_cast<uint32_t>(p)));
+  }
   __device__ __forceinline__ int32_t id(int b, int h, int p) const {
-    const int g = p / T, t = p - g * T;
+    const int g = group(p), t = p - g * T;
     return ids[b * is0 + g * is1 + h * is2 + t * is3];
   }
   __device__ __forceinline__ int limit(int h) const {
     return n_blocks != nullptr ? min(NS, n_blocks[h]) : NS;
   }
   __device__ __forceinline__ int bucket(int32_t bid, int p, int lim) const {
-    const int g = p / T;
     if (bid < 0 || bid >= lim) return -1;
-    // 32-bit unsigned: bid * bs < N + bs and g * G < M + G, with M, N < 2^31
-    if (causal && (static_cast<uint32_t>(bid) * static_cast<uint32_t>(bs)) / static_cast<uint32_t>(chunk) >
-                      (static_cast<uint32_t>(g) * static_cast<uint32_t>(G)) / static_cast<uint32_t>(chunk))
-      return -1;
+    if (causal) {
+      // 32-bit unsigned: bid * bs < N + bs and g * G < M + G, with M, N < 2^31.  The block's chunk
+      // is past the group's when it begins at or after that chunk's end.
+      const uint32_t c = by_chunk(static_cast<uint32_t>(group(p)) * static_cast<uint32_t>(G));
+      if (static_cast<uint32_t>(bid) * static_cast<uint32_t>(bs) >=
+          static_cast<uint64_t>(c + 1) * static_cast<uint32_t>(chunk))
+        return -1;
+    }
     return bid;
   }
 };
@@ -513,12 +538,20 @@ __device__ __forceinline__ void wave_sync_lds() {
 
 // offsets: [B*H][NS+1]; groups: [B*H][MG*T] (bucket j of row r is groups[r][offsets[r][j] ..
 // offsets[r][j+1]), ascending (group, slot)).  One workgroup per (row, 64 buckets lo .. lo+63):
-// wave w of 8 takes the w-th eighth of the row's pairs in order.  Pass 1 counts, per wave, the pairs
+// wave w of 16 takes the w-th sixteenth of the row's pairs in order.  Pass 1 counts, per wave, the pairs
 // of each of the workgroup's buckets and those below lo; the scan then gives every bucket its
 // offset and every (wave, bucket) its first place.  Pass 2 walks each wave's pairs 64 at a time;
 // a pair's place is its (wave, bucket) cursor plus the number of lower lanes of the batch in the
 // same bucket, read from a 64-bit per-(wave, bucket) mask.  Waves touch only their own counters
 // and masks, so the passes need no workgroup barrier inside.
+//
+// Every workgroup of a row looks at all its pairs, and few are of its own buckets (one in 18 of the
+// 34944 of a 32760-token head at 30-token blocks and 15-query groups), so the kernel is bound by
+// the vector work per pair of pass 1: its divisions are multiplications, and pass 1 lists the pairs
+// of the workgroup's buckets (pair and bucket in 32 bits), so that pass 2 walks the lists and not
+// the pairs.  A wave with more than kIdxList of them, or a row of 2^26 pairs or more, walks the
+// pairs again.  Against 8 waves that walked them twice and divided, that shape with 12 heads:
+// 86 -> 42 us; 64-token blocks and 64-query groups: 24 -> 11 us.
 __global__ __launch_bounds__(kIdxThreads) void sel_bwd_index_kernel(
     PairBucket pb, int H, int P, int nrange, int32_t* __restrict__ offsets,
     int32_t* __restrict__ groups) {
@@ -526,6 +559,7 @@ __global__ __launch_bounds__(kIdxThreads) void sel_bwd_index_kernel(
   static_assert(R == kWave, "one bucket per lane in the scan");
   __shared__ int cur[NW][R];                   // counts, then cursors
   __shared__ unsigned long long msk[NW][R];
+  __shared__ uint32_t list[NW][kIdxList];
   __shared__ int below[NW];
   const int row = static_cast<int>(blockIdx.x) / nrange;
   const int rg = static_cast<int>(blockIdx.x) - row * nrange;
@@ -543,9 +577,14 @@ __global__ __launch_bounds__(kIdxThreads) void sel_bwd_index_kernel(
   auto load = [&](int c0, int (&kk)[PL]) {
     int32_t raw[PL];
 #pragma unroll
-    for (int j = 0; j < PL; ++j) raw[j] = pb.id(b, h, min(c0 + j * kWave + lane, p1 - 1));
+    for (int j = 0; j < PL; ++j)
+      if (c0 + j * kWave < p1) raw[j] = pb.id(b, h, min(c0 + j * kWave + lane, p1 - 1));
 #pragma unroll
     for (int j = 0; j < PL; ++j) {
+      if (c0 + j * kWave >= p1) {  // wave-uniform
+        kk[j] = -1;
+        continue;
+      }
       const int p = c0 + j * kWave + lane;
       kk[j] = p < p1 ? pb.bucket(raw[j], p, lim) : -1;
     }
@@ -554,15 +593,23 @@ __global__ __launch_bounds__(kIdxThreads) void sel_bwd_index_kernel(
   cur[w][lane] = 0;
   msk[w][lane] = 0ull;
   wave_sync_lds();
-  int nbelow = 0;
+  int nbelow = 0, nl = 0;
   for (int c0 = p0; c0 < p1; c0 += PL * kWave) {
     int kk[PL];
     load(c0, kk);
 #pragma unroll
     for (int j = 0; j < PL; ++j) {
+      if (c0 + j * kWave >= p1) break;  // wave-uniform
       const int k = kk[j];
+      const bool in = k >= lo && k < lo + nb;
       if (k >= 0 && k < lo) ++nbelow;
-      else if (k >= lo && k < lo + nb) atomicAdd(&cur[w][k - lo], 1);
+      if (in) atomicAdd(&cur[w][k - lo], 1);
+      const uint64_t m = __builtin_amdgcn_ballot_w64(in);
+      if (m == 0) continue;  // wave-uniform
+      const int at = nl + __builtin_popcountll(m & ((1ull << lane) - 1ull));
+      if (in && at < kIdxList)
+        list[w][at] = static_cast<uint32_t>(c0 + j * kWave + lane) << 6 | static_cast<uint32_t>(k - lo);
+      nl += __builtin_popcountll(m);
     }
   }
 #pragma unroll
@@ -595,30 +642,40 @@ __global__ __launch_bounds__(kIdxThreads) void sel_bwd_index_kernel(
   }
   __syncthreads();
 
+  // places 64 pairs in order; a lane's pair p is of bucket k, or of none when k < 0
+  auto place = [&](int k, int p) {
+    const bool in = k >= 0;
+    if (in) atomicOr(&msk[w][k], 1ull << lane);
+    wave_sync_lds();
+    unsigned long long m = 0ull;
+    int r = 0;
+    if (in) {
+      m = msk[w][k];
+      r = __builtin_popcountll(m & ((1ull << lane) - 1ull));
+      grp[cur[w][k] + r] = pb.group(p);
+    }
+    wave_sync_lds();
+    if (in && r == 0) {
+      cur[w][k] += __builtin_popcountll(m);
+      msk[w][k] = 0ull;
+    }
+    wave_sync_lds();
+  };
+  if (nl <= kIdxList && P < (1 << 26)) {  // wave-uniform
+    for (int i = 0; i < nl; i += kWave) {
+      const uint32_t e = i + lane < nl ? list[w][i + lane] : 0u;
+      place(i + lane < nl ? static_cast<int>(e & 63u) : -1, static_cast<int>(e >> 6));
+    }
+    return;
+  }
   for (int c0 = p0; c0 < p1; c0 += PL * kWave) {
     int kk[PL];
     load(c0, kk);
 #pragma unroll
     for (int j = 0; j < PL; ++j) {
       if (c0 + j * kWave >= p1) break;  // wave-uniform
-      const int p = c0 + j * kWave + lane;
-      const int k = kk[j] >= 0 ? kk[j] - lo : -1;
-      const bool in = k >= 0 && k < nb;
-      if (in) atomicOr(&msk[w][k], 1ull << lane);
-      wave_sync_lds();
-      unsigned long long m = 0ull;
-      int r = 0;
-      if (in) {
-        m = msk[w][k];
-        r = __builtin_popcountll(m & ((1ull << lane) - 1ull));
-        grp[cur[w][k] + r] = p / pb.T;
-      }
-      wave_sync_lds();
-      if (in && r == 0) {
-        cur[w][k] += __builtin_popcountll(m);
-        msk[w][k] = 0ull;
-      }
-      wave_sync_lds();
+      const int k = kk[j] - lo;
+      place(kk[j] >= 0 && k >= 0 && k < nb ? k : -1, c0 + j * kWave + lane);
     }
   }
 }
@@ -1706,7 +1763,8 @@ int sel_bwd_launch(const BwdArgs& a, char* ws, const BwdWs& L, hipStream_t s) {
   if (rc) return rc;
 
   PairBucket pb{static_cast<const int32_t*>(ids.data), ids.stride[0], ids.stride[1],
-                ids.stride[2], ids.stride[3], T, NS, bs, ch, G, causal, nullptr};
+                ids.stride[2], ids.stride[3], T, NS, bs, ch, G, causal, nullptr,
+                FastDiv(static_cast<uint32_t>(std::max(T, 1))), FastDiv(static_cast<uint32_t>(std::max(ch, 1)))};
   const int nrange = std::max(1, (NS + kIdxBuckets - 1) / kIdxBuckets);  // NS = 0: offsets[0] = 0
   sel_bwd_index_kernel<<<static_cast<unsigned>(B * H * nrange), kIdxThreads, 0, s>>>(
       pb, H, MG * T, nrange, offsets, groups);
@@ -1780,7 +1838,8 @@ int sel_bwd_ptr_launch(const PtrBwdArgs& a, char* ws, const BwdWs& L, hipStream_
   if (rc || !a.dkv || kv_items == 0) return rc;
 
   PairBucket pb{static_cast<const int32_t*>(ids.data), ids.stride[0], ids.stride[1],
-                ids.stride[2], ids.stride[3], T, NS, a.bs, 1, G, false, a.kg.n_blocks};
+                ids.stride[2], ids.stride[3], T, NS, a.bs, 1, G, false, a.kg.n_blocks,
+                FastDiv(static_cast<uint32_t>(std::max(T, 1))), FastDiv(1)};
   const int nrange = (NS + kIdxBuckets - 1) / kIdxBuckets;
   sel_bwd_index_kernel<<<static_cast<unsigned>(B * H * nrange), kIdxThreads, 0, s>>>(
       pb, H, MG * T, nrange, offsets, groups);

@@ -149,6 +149,26 @@ def test_sel_bwd_f32_block_and_group_edges(BS, G, D):
         _close(name, got, w, *TOL[torch.float32])
 
 
+@pytest.mark.parametrize("BS", [2, 4])
+@pytest.mark.parametrize("M,T", [(2040, 4), (2048, 4), (2100, 4), (700, 13)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_sel_bwd_index_pair_lists(BS, M, T, causal):
+    """The block index's pair lists: 512 pairs of one 64-block range per wave and just below and
+    above (BS 4: one range), two ranges (BS 2), a slot count and a chunk that are no power of two."""
+    N, H, D, G, chunk = 210, 1, 64, 1, 30
+    gen = torch.Generator().manual_seed(M + BS)
+    q, k, v = (torch.randn((1, L, H, D), generator=gen).bfloat16() for L in (M, N, N))
+    ids = torch.randint(0, -(-N // BS), (1, M, H, T), generator=gen, dtype=torch.int32)
+    out, lse, do, dq, dk, dv, scale = _run(q, k, v, ids, G, BS, causal, chunk, torch.bfloat16)
+    want = O.selection_attention_bwd(q.double().numpy(), k.double().numpy(), v.double().numpy(),
+                                     ids.numpy(), out.double().cpu().numpy(),
+                                     lse.double().cpu().numpy(), do.double().numpy(), G, scale,
+                                     O.dense_block_tokens(N, BS, chunk, causal), chunk_size=chunk,
+                                     causal=causal)
+    for name, got, w in (("dq", dq, want[0]), ("dk", dk, want[1]), ("dv", dv, want[2])):
+        _close(name, got, w)
+
+
 # fp32 everywhere; bf16 only at head dims the MFMA kernels do not take (bf16 at 64 / 128 runs
 # the MFMA kernels, covered by test_sel_bwd_matches_oracle)
 VALU_PARAMS = [pytest.param(case, dt, id=f"valu{i}-{'f32' if dt == torch.float32 else 'bf16'}")
