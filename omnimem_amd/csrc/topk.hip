@@ -1663,6 +1663,9 @@ constexpr int kExSpanCap = 1792;  // columns per item: 28 a lane, 115 KiB of sco
 constexpr int kExCand = 128;      // candidates per row, two a lane
 constexpr int kExMaxTopk = 64;
 constexpr float kExNorm2Min = 1e-30f, kExNorm2Max = 1e30f;
+// E is 3e-5 |q| max |k| |scale| at D = 128: the scores stay far below overflow, and E far above what
+// denormal products could lose (128 of 1.2e-38)
+constexpr float kExBoundMin = 1e-30f, kExBoundMax = 1e25f;
 
 __host__ __device__ inline int ex_pitch(int span) { return span + 4; }  // span: a multiple of 16
 inline size_t ex_lds_bytes(int span, int D) {
@@ -1829,7 +1832,7 @@ __global__ __launch_bounds__(kExThreads) void topk_exact_kernel(M2Args a) {
   const float q2 = qn2[r], k2 = __builtin_bit_cast(float, kn2);
   const float E = 4.0f * D * 0x1p-24f * __builtin_sqrtf(q2) * __builtin_sqrtf(k2) * fabsf(a.scale);
   bool ok = kbad == 0 && q2 >= kExNorm2Min && q2 <= kExNorm2Max && k2 >= kExNorm2Min &&
-            fabsf(a.scale) >= 1e-6f && fabsf(a.scale) <= 1e10f;
+            E >= kExBoundMin && E <= kExBoundMax;
   uint16_t* const list = reinterpret_cast<uint16_t*>(sv + kExCand);  // behind the candidates' keys
   int nc = 0;
   if (ok && nvis > 0) {

@@ -431,6 +431,18 @@ def test_topk_exact_preselection_matches_general_path(dtype, data, T, NC, H, D, 
             got.cpu().numpy(), O.topk(O.pool_mean(_img(q), G, name), _img(k), topk, D ** -0.5, mask))
 
 
+@pytest.mark.parametrize("scale", [0.0, -0.5, 1e-30, 1e30, float("inf"), float("nan")])
+def test_topk_exact_preselection_scales(scale):
+    """Scales whose scores overflow or leave the normal range, and the ones without an order."""
+    from omnimem_amd.index_topk import parallel_nsa_topk
+    g = torch.Generator().manual_seed(7)
+    q, k = (_bf16((1, L, 2, 128), g).to(DEV) for L in (400, 600))
+    odd = torch.zeros((1, 600, 2, 129), dtype=k.dtype, device=DEV)[..., :128]
+    odd.copy_(k)
+    kw = dict(block_size=4, chunk_size=100, causal=False, group_size=4, scale=scale)
+    assert torch.equal(parallel_nsa_topk(q, k, 40, **kw), parallel_nsa_topk(q, odd, 40, **kw))
+
+
 # Mask modes on the MFMA path's four-rows-per-wave selection, whose visibility is a pair of
 # column intervals per row (one visible run, plus a noisy row's own noisy chunk under tf_mask or
 # the chunks past a non-causal exclusion window).  Each case is (T, NC, H, D, G, topk, facade
