@@ -3,8 +3,8 @@
 Reference: src/omnimem/nsa/ops/selection/__init__.py:12-100 (facade and validation),
 cuda_backend/ops.py:90-117 (op adapters) and cuda_backend/autograd.py:9-45 (autograd wiring:
 the forward saves q, k, v, ids, out and lse; the backward returns dq, dk, dv).  The backward
-runs on gfx950 MFMA for bf16 / f16 with head dim 64 or 128, and on fp32 VALU kernels for fp32
-and every other head dim up to 256.
+runs on gfx950 MFMA for bf16 / f16 / fp32 with head dim 64 or 128 (fp32 on the fp32 matrix
+instructions), and on fp32 vector kernels for every other head dim up to 256.
 Extension: ``M % group_size`` need not be 0 (the last query group may be ragged).
 """
 from __future__ import annotations
