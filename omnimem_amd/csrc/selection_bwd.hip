@@ -10,8 +10,9 @@
 // in the K / V dtype).
 //
 // gfx950 design (bf16 / f16; fp32 in the same three launches on its own MFMA kernels):
-//   sel_bwd_dq_kernel    one workgroup = 64 queries of one group, 2 waves x 32 queries, the same
-//                        block walk and LDS-DMA K / V tiles as the forward kernel.  Per key tile:
+//   sel_bwd_dq_kernel    one workgroup = 64 queries of one group, 2 waves x 32 queries (groups of
+//                        at most 32: sel_bwd_dq_wave_kernel, one wave), the same block walk and
+//                        LDS-DMA K / V tiles as the forward kernel.  Per key tile:
 //                        S^T = K Q^T and dP^T = V dO^T (K and V rows from LDS, Q^T and dO^T held
 //                        in registers), P = 2^(s c2 - lse log2 e), dS = P (dP - delta) scale,
 //                        then dQ^T += K^T dS^T with dS^T straight from the accumulator layout and
@@ -20,10 +21,11 @@
 //                        valid (group, slot) pair into per-block buckets (CSR), in (group, slot) order,
 //                        so the dK / dV sums have a fixed order (the reference's buckets are in
 //                        atomic arrival order).
-//   sel_bwd_dkv_kernel   one workgroup per (b, h, block, 64-key tile), 2 waves x 32 keys.  K and V
-//                        of its keys stay in registers as MFMA operands; the queries of each
-//                        bucket group stream through LDS (64-row Q / dO tiles by LDS DMA, double
-//                        buffered, with their lse and delta).  S = Q K^T, dP = dO V^T, then
+//   sel_bwd_dkv_kernel   one workgroup per (b, h, block, 64-key tile), 4 waves x 16 keys (32-key
+//                        tiles and 2 waves for small blocks).  K and V of its keys stay in
+//                        registers as MFMA operands; the queries of the bucket's groups stream
+//                        through LDS (16 NW-row Q / dO tiles by LDS DMA, double buffered, with
+//                        their lse and delta; small groups share a tile).  S = Q K^T, dP = dO V^T, then
 //                        dV += P^T dO and dK += dS^T Q with P^T / dS^T from the accumulator
 //                        layout and dO / Q from transposed LDS reads.  Every token of every block
 //                        is written (0 when no group selected it).
@@ -1103,9 +1105,10 @@ __global__ __launch_bounds__(NW * kWave, 2) void sel_bwd_dkv_kernel(
 // l16, chunk 4 u + j4: the dims 16 u + 4 j4 + e of the k-steps 4 u + e, four of them a read) and
 // transposed ones (rows 4 j4 + r, dim 16 i + l16, one a read).  Against the VALU kernels, which
 // reread every LDS operand for each of 4 lanes and had one workgroup per query group: 1560 queries
-// over 16 blocks of 64 of 4680 keys, 12 heads, head dim 128: dQ 2171 -> 190 us, dK / dV 763 -> 248 us (94
-// and 125 us at the fp32 matrix rate); 3900 tokens over themselves 5560 -> 982 us for the whole
-// backward, with blocks of 30 and groups of 15 7900 -> 560.
+// over 16 blocks of 64 of 4680 keys, 12 heads, head dim 128: dQ 2171 -> 204 us, dK / dV 763 -> 272 us
+// (94 and 125 us at the fp32 matrix rate).  Error against 64 bits there, VALU and now: dQ 7.1e-7 and
+// 5.1e-7, dK 5.4e-7 both, dV 5.3e-7 both; S and dP in one chain of D products and P as a plain 2^x of
+// -lse log2 e + s c2 took 190 and 248 us but had 6.4e-7, 6.7e-7 and 6.5e-7.
 template <int D>
 struct F32Tile {
   static constexpr int ROWB = 4 * D, CPR = D / 4, RPI = 1024 / ROWB;
@@ -1135,13 +1138,36 @@ __device__ __forceinline__ f32x4 mfma4(const float4& a, const float4& b, f32x4 c
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b.w, c, 0, 0, 0);
 }
 
-// dQ (and delta, -lse log2 e) of 16 queries of one group: 4 waves that take every fourth 16-key tile
+// S or dP of a tile: rows of LDS against the lane's operands, in four chains of D / 4 products, whose
+// sum is closer than one chain's and whose instructions need not wait for each other.
+template <int DU>
+__device__ __forceinline__ f32x4 dot_rows(const char* tile, int rb, const float4 (&x)[DU]) {
+  f32x4 c[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) c[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int u = 0; u < DU; ++u)
+    c[u & 3] = mfma4(*reinterpret_cast<const float4*>(tile + (rb ^ (u << 6))), x[u], c[u & 3]);
+  return (c[0] + c[1]) + (c[2] + c[3]);
+}
+
+// e^x: 2^y of y = x log2 e, times the first order of what y's rounding and log2 e's own leave out.
+__device__ __forceinline__ float exp_nat(float x) {
+  constexpr float kLog2eLo = 1.9259629911e-8f;  // log2 e - kLog2e
+  constexpr float kLn2 = 0.693147181f;
+  const float y = x * kLog2e;
+  const float p = __builtin_amdgcn_exp2f(y);
+  const float r = __builtin_fmaf(x, kLog2eLo, __builtin_fmaf(x, kLog2e, -y)) * kLn2;
+  return p > 0.0f ? __builtin_fmaf(p, r, p) : p;  // (x = -inf leaves r undefined)
+}
+
+// dQ (and delta, -lse) of 16 queries of one group: 4 waves that take every fourth 16-key tile
 // of the group's blocks, each in its own LDS buffers, so that a call of a few hundred groups fills
 // the CUs; their sums are added in wave order at the end.
 template <typename Acc, int D>
 __global__ __launch_bounds__(256, 2) void sel_bwd_dq_f32_kernel(
     View4<const float> q, View4<const float> o, View4<const float> dout, View4<float> dq,
-    const float* __restrict__ lse, float* __restrict__ delta, float* __restrict__ nl2out, Acc acc,
+    const float* __restrict__ lse, float* __restrict__ delta, float* __restrict__ nlout, Acc acc,
     int M, int H, int G, int MG, int T, int chunk, float scale, int nsub) {
   using FT = F32Tile<D>;
   constexpr int DU = FT::DU, NI = FT::NI;
@@ -1176,12 +1202,13 @@ __global__ __launch_bounds__(256, 2) void sel_bwd_dq_f32_kernel(
   dl += __shfl_xor(dl, 16, kWave);
   dl += __shfl_xor(dl, 32, kWave);
   const int64_t li = (static_cast<int64_t>(b) * H + h) * M + mq;
-  const float nl2 = q_ok ? neg_lse2(lse[li]) : kNegInf;
+  // -lse in the natural log: its product with log2 e, rounded, would put 3e-7 on every P of the row
+  const float lrow = q_ok ? lse[li] : kNegInf;
+  const float nl = lrow == kNegInf ? kNegInf : -lrow;
   if (w == 0 && q_ok && j4 == 0) {
     delta[li] = dl;
-    nl2out[li] = nl2;
+    nlout[li] = nl;
   }
-  const float c2 = scale * kLog2e;
   const int rb = FT::rb();
   int tb[4];
 #pragma unroll
@@ -1223,18 +1250,12 @@ __global__ __launch_bounds__(256, 2) void sel_bwd_dq_f32_kernel(
   while (wk.valid) {
     const int n = wk.n;
     // S^T = K Q^T and dP^T = V dO^T: lane holds keys 4 j4 + r of query l16
-    f32x4 s4 = f32x4{0.f, 0.f, 0.f, 0.f}, p4 = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int u = 0; u < DU; ++u)
-      s4 = mfma4(*reinterpret_cast<const float4*>(kbuf + (rb ^ (u << 6))), qf[u], s4);
-#pragma unroll
-    for (int u = 0; u < DU; ++u)
-      p4 = mfma4(*reinterpret_cast<const float4*>(vbuf + (rb ^ (u << 6))), df[u], p4);
+    const f32x4 s4 = dot_rows<DU>(kbuf, rb, qf), p4 = dot_rows<DU>(vbuf, rb, df);
     // dS / scale = P (dP - delta); keys past n are not visible
     float ds[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const float p = 4 * j4 + r < n ? __builtin_amdgcn_exp2f(__builtin_fmaf(s4[r], c2, nl2)) : 0.0f;
+      const float p = 4 * j4 + r < n ? exp_nat(__builtin_fmaf(s4[r], scale, nl)) : 0.0f;
       ds[r] = p * (p4[r] - dl);
     }
     // dQ^T += K^T dS^T, k-step r: keys 4 j4 + r
@@ -1284,7 +1305,7 @@ __global__ __launch_bounds__(256, 2) void sel_bwd_dq_f32_kernel(
 template <int D, int NW>
 __global__ __launch_bounds__(NW * kWave, 2) void sel_bwd_dkv_f32_kernel(
     View4<const float> q, View4<const float> dout, DenseGrad<float> kg,
-    const float* __restrict__ nl2, const float* __restrict__ delta,
+    const float* __restrict__ nl, const float* __restrict__ delta,
     const int32_t* __restrict__ offsets, const int32_t* __restrict__ groups, int M, int H, int G,
     int MG, int T, int NS, int nkt, int chunk, bool causal, float scale, int nparts) {
   using FT = F32Tile<D>;
@@ -1292,7 +1313,7 @@ __global__ __launch_bounds__(NW * kWave, 2) void sel_bwd_dkv_f32_kernel(
   constexpr int NIW = 2 * FT::NI / NW;  // this wave's copy instructions of a Q and dO tile pair
   static_assert(NIW % 2 == 0, "whole copies of 2 or 4 instructions");
   __shared__ __align__(16) char smem[2][2][FT::BYTES];  // [buffer][Q, dO]
-  __shared__ float rowv[2][2][64];                      // [buffer][-lse log2 e, delta]
+  __shared__ float rowv[2][2][64];                      // [buffer][-lse, delta]
   const int lane = lane_id();
   const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
   const int l16 = lane & 15, j4 = lane >> 4;
@@ -1316,7 +1337,6 @@ __global__ __launch_bounds__(NW * kWave, 2) void sel_bwd_dkv_f32_kernel(
       }
     }
   }
-  const float c2 = scale * kLog2e;
   const int rb = FT::rb();
   int tb[4];
 #pragma unroll
@@ -1375,7 +1395,7 @@ __global__ __launch_bounds__(NW * kWave, 2) void sel_bwd_dkv_f32_kernel(
       dma_part<NIW>(base, rs, it.nq, dst, part, off);
     }
     if (w < 2)
-      dma_f32x64((w == 0 ? nl2 : delta) + lrow + it.q0, lane < it.nq ? 4 * lane : -1,
+      dma_f32x64((w == 0 ? nl : delta) + lrow + it.q0, lane < it.nq ? 4 * lane : -1,
                  rowv[buf][w]);
   };
 
@@ -1392,13 +1412,7 @@ __global__ __launch_bounds__(NW * kWave, 2) void sel_bwd_dkv_f32_kernel(
     const char* Dt = smem[BI][1];
     if (16 * w < cur.nv) {  // wave-uniform
       // S = Q K^T and dP = dO V^T: lane holds queries 4 j4 + r of key 16 w + l16
-      f32x4 s4 = f32x4{0.f, 0.f, 0.f, 0.f}, p4 = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int u = 0; u < DU; ++u)
-        s4 = mfma4(*reinterpret_cast<const float4*>(Qt + (rb ^ (u << 6))), kb[u], s4);
-#pragma unroll
-      for (int u = 0; u < DU; ++u)
-        p4 = mfma4(*reinterpret_cast<const float4*>(Dt + (rb ^ (u << 6))), vb[u], p4);
+      const f32x4 s4 = dot_rows<DU>(Qt, rb, kb), p4 = dot_rows<DU>(Dt, rb, vb);
       const float4 L4 = *reinterpret_cast<const float4*>(rowv[BI][0] + 4 * j4);
       const float4 D4 = *reinterpret_cast<const float4*>(rowv[BI][1] + 4 * j4);
       const float Lr[4] = {L4.x, L4.y, L4.z, L4.w}, Dr[4] = {D4.x, D4.y, D4.z, D4.w};
@@ -1407,7 +1421,7 @@ __global__ __launch_bounds__(NW * kWave, 2) void sel_bwd_dkv_f32_kernel(
       // rows past the item's queries have zero Q / dO and lse = delta = 0, so they add nothing
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        pv[r] = kv ? __builtin_amdgcn_exp2f(__builtin_fmaf(s4[r], c2, Lr[r])) : 0.0f;
+        pv[r] = kv ? exp_nat(__builtin_fmaf(s4[r], scale, Lr[r])) : 0.0f;
         ds[r] = pv[r] * (p4[r] - Dr[r]);
       }
       // dV += P^T dO and dK += dS^T Q, k-step r: queries 4 j4 + r
