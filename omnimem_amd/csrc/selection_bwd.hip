@@ -1105,10 +1105,10 @@ __global__ __launch_bounds__(NW * kWave, 2) void sel_bwd_dkv_kernel(
 // l16, chunk 4 u + j4: the dims 16 u + 4 j4 + e of the k-steps 4 u + e, four of them a read) and
 // transposed ones (rows 4 j4 + r, dim 16 i + l16, one a read).  Against the VALU kernels, which
 // reread every LDS operand for each of 4 lanes and had one workgroup per query group: 1560 queries
-// over 16 blocks of 64 of 4680 keys, 12 heads, head dim 128: dQ 2171 -> 204 us, dK / dV 763 -> 272 us
-// (94 and 125 us at the fp32 matrix rate).  Error against 64 bits there, VALU and now: dQ 7.1e-7 and
-// 5.1e-7, dK 5.4e-7 both, dV 5.3e-7 both; S and dP in one chain of D products and P as a plain 2^x of
-// -lse log2 e + s c2 took 190 and 248 us but had 6.4e-7, 6.7e-7 and 6.5e-7.
+// over 16 blocks of 64 of 4680 keys, 12 heads, head dim 128: dQ 2171 -> 204 us, dK / dV 763 ->
+// 272 us (94 and 125 us at the fp32 matrix rate).  Error against 64 bits there, VALU and now: dQ
+// 7.1e-7 and 5.1e-7, dK 5.4e-7 both, dV 5.3e-7 both; S and dP in one chain of D products and P as a
+// plain 2^x of s c2 - lse log2 e took 190 and 248 us but had 6.4e-7, 6.7e-7 and 6.5e-7.
 template <int D>
 struct F32Tile {
   static constexpr int ROWB = 4 * D, CPR = D / 4, RPI = 1024 / ROWB;
