@@ -167,6 +167,11 @@ struct DenseAcc {
     const uint32_t vo = static_cast<uint32_t>(e.t0) * static_cast<uint32_t>(v.s1);
     return BlockRef{kb + ko, vb + vo, k.s1, v.s1, e.n, 1.0f, 1.0f};
   }
+  // tokens that a query group can list, on average
+  int64_t mean_reach() const {
+    const int64_t c = static_cast<int64_t>(N) + chunk;
+    return causal && c < 2 * static_cast<int64_t>(N) ? c / 2 : N;
+  }
   __device__ __forceinline__ static int64_t order_key(const Ent& e) { return e.t0; }
   __device__ __forceinline__ void touch(int, int, int, int) const {}
 };
@@ -176,7 +181,7 @@ struct PtrAcc {
   // raw caller addresses: any 2-byte alignment is accepted (the reference's contract), so the
   // staging checks each block and copies misaligned ones with 2-byte loads
   static constexpr bool kMayMisalign = true;
-  static constexpr bool kHistory = true;  // blocks of a cache, as many as a long video's
+  static constexpr bool kHistory = true;  // blocks of a cache
   struct Ent {
     int64_t k, v;  // raw addresses (0 = skip)
     int n;
@@ -218,7 +223,7 @@ template <> struct PagedEntOf<uint8_t> { using type = PagedEnt8; };
 template <typename KVT>
 struct PagedAcc {
   static constexpr bool kMayMisalign = false;  // 16-byte rows checked on the host
-  static constexpr bool kHistory = true;  // blocks of a cache, as many as a long video's
+  static constexpr bool kHistory = true;  // blocks of a cache
   using KV = KVT;
   using Ent = typename PagedEntOf<KVT>::type;
   const KVT* pool_k;

@@ -1700,32 +1700,46 @@ inline int device_cus() {
   return n;
 }
 
-// Whether one wave per query group takes a call (sel_fwd_wave_kernel).  A cache call of groups of 17
-// to 32 queries with at most 8 of them per CU keeps the 64-query kernel, which has two tiles in
-// flight: 30-query groups over 60-token blocks, 7.3 per CU, 135.0 against 137.3 us.
-template <typename Acc>
+// Whether one wave per query group takes a call (sel_fwd_wave_kernel).  Its walk of a group's list
+// has one tile in flight and the 64-query kernel's two, which groups of 17 to 32 feel while they
+// have a CU to themselves: 32-query groups over 64-token blocks, half a group to one per CU, 31 us
+// against 27 (30 / 60 33 and 28, 24 / 24 with 64 slots 67 and 58; from 1.5 per CU on no slower, from
+// 6 on 20-40% faster), and with head dim 64, whose copies are half as long, up to 3 (32 / 128 two per
+// CU 24.9 and 23.2 us).  A cache call of such groups keeps the 64-query kernel up to 8 per CU: 60-token
+// blocks of 10 chunks, groups of 30, 7.3 per CU, 103.5 against 110 us.  Groups of at most 16 lose
+// nothing in one wave.
+template <typename Acc, int D>
 bool wave_kernel(const Geom& gm) {
-  return gm.G <= 16 ||
-         (gm.G <= 32 && !(Acc::kHistory && gm.items <= int64_t{8} * device_cus()));
+  constexpr int64_t kPerCu = Acc::kHistory ? 8 : D == 64 ? 3 : 1;
+  return gm.G <= 16 || (gm.G <= 32 && gm.items > kPerCu * device_cus());
 }
 
 template <typename QT, typename Acc, int D>
 int launch_dma(const Geom& gm, const omm_view4& q, const omm_view4& out, float* lse,
                const Acc& acc, int chunk, float scale, hipStream_t s, const GateArgs& gate) {
-  if (wave_kernel<Acc>(gm)) {
-    // A cache's blocks do not fit the memory-side cache, and the fewer groups sweep them at a time
-    // the more of them share a block: 6 waves a CU (by LDS) where the call has more than 8 for
-    // each.  Over 27 chunks of 4680 tokens, 12 heads, top-16: 142 us with 10, 134 with 6, 139 with
-    // the 64-query kernel; top-64 over blocks and groups of 24 262, 225 and 265 us.  (Of a clip,
-    // which fits, more waves are better: 458 us with 6, 450 with 10; head dim 64 196 and 165.)
-    const bool few = Acc::kHistory && gm.items > int64_t{8} * device_cus();
+  if (wave_kernel<Acc, D>(gm)) {
+    // What a call with more than 8 groups per CU misses in L2 depends on how many sweep a head's
+    // blocks at a time, and two things hold that down.
+    const bool many = gm.items > int64_t{8} * device_cus();
+    // 6 waves a CU (by LDS), where a head's K and V are far more than an XCD's 4 MiB of L2: over
+    // 27 chunks of 4680 tokens, 12 heads, top-16, blocks of 30, groups of 15 142 us with 10 waves,
+    // 134 with 6; 24 / 24 with 64 slots 262 and 225; five chunks 97 and 81.  Calls of any head count
+    // turn at the same size of a head, 10 MB: blocks of 30, groups of 15 over 16380 tokens (8.4 MB)
+    // 212 us with 10 waves, 216 with 6; 20000 314 and 291; 32760 690 and 617 (680 with the 64-query
+    // kernel).  A causal clip reaches half of it on average (454 and 468); groups of 17 to 32 over a
+    // clip read half as much and keep 10 (24 / 24 with 64 slots over 32760 tokens 966 and 1232).  A
+    // cache with less keeps 6 for its counters' sake (3 chunks, head dim 64: 77 and 70 us).
+    bool few = many;
+    if constexpr (!Acc::kHistory)
+      few = many && gm.G <= 16 && acc.mean_reach() * (4 * D) > 10000000;
     const size_t lds = few ? 27000 - 2 * WaveTile<Acc, D>::BYTES : 0;
-    // Waiting for the next tile's copies before this tile's S keeps fewer in flight, which short
-    // lists over a clip share better in L2: blocks of 30, groups of 15 450 us, waiting at the end
-    // 458 (16380 tokens 160 and 167; 60 / 30 384 and 400).  Long lists and caches wait at the end:
-    // top-64 over 24 / 24 735 us against 752 (4680 tokens 147 and 157; a cache of 27 chunks 225
-    // and 242).
-    const bool early = !Acc::kHistory && gm.T <= 32;
+    // Waiting for the next tile's copies before this tile's S keeps fewer of them in flight: over a
+    // clip, blocks of 30, groups of 15 464 us, waiting before S 454 (60 / 30 398 and 382; 16380
+    // tokens, every block visible, 238 and 212, with 48 slots 625 and 508).  With few groups there is
+    // nothing to share and the wait is bare latency (30 / 60, one per CU: 33 and 39 us).  Long lists of
+    // larger groups and caches wait at the end: 24 / 24 with 64 slots 737 us against 772 (4680
+    // tokens 148 and 157, with 32 slots 80 and 85; a cache of 27 chunks 225 and 242).
+    const bool early = !Acc::kHistory && many && gm.T <= 32;
     const unsigned grid = static_cast<unsigned>(gm.items);
     if (gm.G <= 16)
       sel_fwd_wave_kernel<QT, Acc, D, 1><<<grid, kWave, lds, s>>>(

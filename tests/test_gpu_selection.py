@@ -106,6 +106,38 @@ def test_sel_fwd_small_group_edges(BS, G, D, scale):
     _check(out, lse, want_o, want_l, torch.bfloat16)
 
 
+@pytest.mark.parametrize("G,D,BS,T,N,per_cu", [
+    # a group to each CU (head dim 64: three): the 64-query kernel; more: one wave, two row blocks
+    (17, 64, 33, 5, 333, 0), (32, 128, 64, 5, 333, 0), (30, 128, 65, 5, 333, 1),
+    (32, 128, 32, 5, 333, 1), (30, 64, 65, 5, 333, 2), (17, 64, 30, 67, 1900, 3),
+    (31, 64, 16, 5, 333, 3),
+    (17, 128, 30, 33, 990, 8), (32, 64, 33, 5, 333, 8),  # more than 8: waits before S up to 32 slots
+    (1, 64, 24, 3, 40000, 8), (15, 64, 30, 3, 40000, 8), (16, 128, 64, 3, 20000, 8),  # fewer waves
+])
+def test_sel_fwd_one_wave_dispatch_edges(G, D, BS, T, N, per_cu):
+    """Either side of the group counts (per CU) and the K / V size where the one-wave kernel takes
+    over, waits earlier and runs fewer waves, with -1 and out-of-range ids, causal prefixes that cut
+    blocks and a ragged last group."""
+    from omnimem_amd.selection import sel_fwd
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    H = 8
+    MG = max(per_cu, 1) * cus // H + (1 if per_cu else 0)
+    M = MG * G - (1 if G > 1 else 0)
+    chunk = 2 * M if N >= 20000 else 60 * G
+    gen = torch.Generator().manual_seed(BS * 100 + G)
+    q = (torch.randn((1, M, H, D), generator=gen) * D ** -0.25).bfloat16()
+    k = (torch.randn((1, N, H, D), generator=gen) * D ** -0.25).bfloat16()
+    v = torch.randn((1, N, H, D), generator=gen).bfloat16()
+    ids = _ids(gen, 1, MG, H, T, -(-N // BS) + 1, 0.2)
+    causal = N < 20000
+    out, lse = sel_fwd(q.to(DEV), k.to(DEV), v.to(DEV), ids.to(DEV), BS, chunk, D ** -0.5, causal, G)
+    want_o, want_l = O.selection_attention(q.float().numpy(), k.float().numpy(), v.float().numpy(),
+                                           ids.numpy(), G, D ** -0.5,
+                                           O.dense_block_tokens(N, BS, chunk, causal),
+                                           chunk_size=chunk, causal=causal)
+    _check(out, lse, want_o, want_l, torch.bfloat16)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("scale", [-0.09, 0.0, 8.0])
 def test_sel_fwd_scale_values(scale, dtype):
