@@ -1111,3 +1111,88 @@ def test_selection_counters_match_the_listings(n_chunks, G, T):
     np.testing.assert_array_equal(cache.touches[0].cpu().numpy(), calls)
     np.testing.assert_array_equal(cache.seen[0].cpu().numpy(), seen)
     cache.close()
+
+
+@pytest.mark.parametrize("G,D,BS,T", [(15, 64, 30, 3), (17, 64, 33, 3), (30, 128, 24, 3), (32, 64, 65, 67)])
+@pytest.mark.parametrize("shift", [0, 1, 4])
+def test_padded_ptr_many_small_groups(G, D, BS, T, shift):
+    """More groups than 8 per CU, where one wave takes a group of up to 32 queries over addresses
+    (one or two row blocks, fewer waves), with chunk bases on 16, 2 and 8 bytes and head 1 mixing
+    them, blocks shorter and longer than its 32-key tiles and a skipped chunk."""
+    from omnimem_amd.padded_ptr import selection_attention_padded_ptr_fast
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    H, bpc, n_chunks = 16, 12, 3
+    C, MG = bpc * BS, 8 * cus // 16 + 1
+    M = MG * G
+    g = torch.Generator().manual_seed(G + shift)
+
+    def chunk(i, scale):
+        x = (torch.randn((1, C * D + 8), generator=g) * scale).to(torch.bfloat16).to(DEV)
+        off = shift if i % 2 == 0 else 0
+        return x[:, off:off + C * D].view(1, C, D)
+
+    chunks_k = [[chunk(h + c, 0.3) for c in range(n_chunks)] for h in range(H)]
+    chunks_v = [[chunk(h + c + 1, 1.0) for c in range(n_chunks)] for h in range(H)]
+    base_k = torch.tensor([[t.data_ptr() for t in row] for row in chunks_k], dtype=torch.int64)
+    base_v = torch.tensor([[t.data_ptr() for t in row] for row in chunks_v], dtype=torch.int64)
+    assert bool(((base_k % 16) != 0).any()) == (shift != 0)
+    base_k[1, 0] = 0
+    q = (torch.randn((1, M, H, D), generator=g) * 0.3).to(torch.bfloat16)
+    ids = torch.randint(-1, n_chunks * bpc, (1, MG, H, T), generator=g, dtype=torch.int32)
+    strides = {"batch_stride_bytes": C * D * 2, "token_stride_bytes": D * 2, "stride_bn": D,
+               "stride_bd": 1, "chunk_len": C}
+    out, lse = selection_attention_padded_ptr_fast(
+        q.to(DEV), ids.to(DEV), BS, G, C, base_k.to(DEV), base_v.to(DEV),
+        torch.full((H,), n_chunks, dtype=torch.int32, device=DEV), strides, return_lse=True)
+    k = torch.stack([torch.cat([c[0] for c in row]) for row in chunks_k], 1)[None].float().cpu()
+    v = torch.stack([torch.cat([c[0] for c in row]) for row in chunks_v], 1)[None].float().cpu()
+    ids_np = ids.numpy().copy()
+    ids_np[:, :, 1][ids_np[:, :, 1] // bpc == 0] = -1
+    want_o, want_l = O.selection_attention(q.float().numpy(), k.numpy(), v.numpy(), ids_np, G,
+                                           D ** -0.5, O.dense_block_tokens(n_chunks * C, BS, 1, False))
+    _check_attn(out, lse, want_o, want_l)
+
+
+@pytest.mark.parametrize("G,D,P,T", [(15, 64, 30, 3), (16, 128, 64, 3), (17, 64, 33, 3), (30, 128, 24, 3),
+                                     (32, 64, 16, 67)])
+def test_paged_many_small_groups(G, D, P, T):
+    """More groups than 8 per CU over the paged cache, plain and with the gated mix in the one-wave
+    kernel's epilogue, pages in HBM and on the host, a short last page and group, and the counters."""
+    from omnimem_amd.block_cache import PagedKVCache
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    H, n = 16, 3
+    C, MG = 5 * P - 3, 8 * cus // 16 + 1
+    M = MG * G - 1
+    g = torch.Generator().manual_seed(G)
+    cache = PagedKVCache(1, H, D, max_chunks=n, chunk_len=C, page_tokens=P, hbm_slots=H * n,
+                         host_slots=H * n, window_chunks=0)
+    ks = [_chunk(g, C, H, D, 0.3) for _ in range(n)]
+    vs = [_chunk(g, C, H, D, 1.0) for _ in range(n)]
+    for cid in range(n):
+        cache.append(0, ks[cid].to(DEV), vs[cid].to(DEV), cid)
+    q = (torch.randn((1, M, H, D), generator=g) * 0.3).to(torch.bfloat16)
+    ids = torch.randint(-1, n * cache.ppc + 1, (1, MG, H, T), generator=g, dtype=torch.int32)
+    gates = torch.sigmoid(torch.randn((1, M, H, 3), generator=g) * 2).to(torch.bfloat16)
+    o_cmp, o_swa = (torch.randn((1, M, H, D), generator=g).to(torch.bfloat16) for _ in range(2))
+    qd, idd = q.to(DEV), ids.to(DEV)
+    plain, lse = cache.select(qd, idd, 0, G, return_lse=True)
+    want_o, want_l = O.selection_attention(q.float().numpy(), torch.cat(ks, 1).float().numpy(),
+                                           torch.cat(vs, 1).float().numpy(), ids.numpy(), G,
+                                           D ** -0.5, O.paged_block_tokens(C, P, n))
+    _check_attn(plain, lse, want_o, want_l)
+    reads = np.zeros((H, n), dtype=np.int64)
+    for h in range(H):
+        x = ids[0, :, h].numpy().ravel()
+        np.add.at(reads[h], x[(x >= 0) & (x < n * cache.ppc)] // cache.ppc, 1)
+    np.testing.assert_array_equal(cache.reads[0].cpu().numpy(), reads)
+    np.testing.assert_array_equal(cache.touches[0].cpu().numpy(), np.ones((H, n)))
+    cache.evict_all()
+    mix, lse2 = cache.select(qd, idd, 0, G, gates=gates.to(DEV), o_cmp=o_cmp.to(DEV),
+                             o_swa=o_swa.to(DEV), return_lse=True)
+    assert torch.equal(lse, lse2)
+    gg = gates.float().numpy().astype(np.float64)
+    want = (gg[..., 0:1] * o_cmp.float().numpy() + gg[..., 1:2] * want_o
+            + gg[..., 2:3] * o_swa.float().numpy())
+    # O(1) mixes: their bf16 rounding alone is about 1e-3 mean-abs
+    _check_attn(mix, lse2, want, want_l, mx=4e-2, mean=3e-3)
+    cache.close()
