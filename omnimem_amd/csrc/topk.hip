@@ -142,10 +142,19 @@ constexpr int kMaxPer = kSpanCap / kWave;
 // Up to this topk theta comes from the 64 lane maxima, past it from an exact radix select.  The
 // lane maxima cost less, but close to 64 they cut almost nothing: with 16 keys a lane the 56th
 // largest of the 64 maxima leaves about 125 survivors, the 64th (their minimum) about 300, past
-// the survivor buffer, and the row then takes its maxima one at a time.  16380 rows of 1365
-// columns: topk 56 285 us with the maxima and 292 us with the radix select, topk 64 558 and 295 us
-// (4680 tokens over 5920 columns: 119 and 117 us, 283 and 118 us).
+// the survivor buffer, and the row then takes its maxima one at a time.  4000 rows of 1024 scores:
+// topk 57 88 us with the maxima and 77 with the radix select, topk 64 114 and 77.
 constexpr int kLaneMaxTopk = 56;
+// Up to 64, rows of so few visible keys (one or two a lane) keep the lane maxima: they leave few
+// survivors more than the radix select's (4000 rows of 64 scores 14.7 and 19.5 us, of 128 25 and 20;
+// 64 causal fp32 rows of 3000 columns, 12 heads 36 and 43 us).
+constexpr int kLaneMaxFew = 96;
+// The merge of many column spans reads its keys again on every pass, so the radix select's four
+// cost more there: 40 rows of 5000 scores in spans of 128, topk 57 42 us with the maxima and 62 with
+// the radix select, topk 60 47 and 65.  Past 60 the maxima leave too many (topk 64 404 and 67), but
+// for rows whose spans are mostly hidden: as many keys as the survivor buffer holds need no
+// threshold (64 causal rows of 3000 columns, topk 64: 37 us without one and 56).
+constexpr int kLaneMaxTopkStream = 60;
 
 // Wave-wide max of an unsigned value (DPP row shifts and row broadcasts; every lane gets it).
 template <int CTRL, int ROW_MASK>
@@ -271,7 +280,14 @@ __device__ __forceinline__ void wave_select_impl(int n, int topk, KeyF key, Emit
   }
   // theta: the topk-th largest lane maximum (0 if fewer than topk lanes hold candidates), or the
   // exact topk-th largest high word
-  const uint32_t theta = topk <= kLaneMaxTopk
+  bool maxima = topk <= kLaneMaxTopk;
+  if (!maxima && topk <= kWave) {  // wave-uniform
+    int live = 0;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) live += popc64(ballot64(kv[j] != 0ull));
+    maxima = live <= kLaneMaxFew;
+  }
+  const uint32_t theta = maxima
       ? lane_max_threshold(lmax, topk, reinterpret_cast<uint32_t*>(sv))
       : wave_radix_threshold(
             PER, topk,
@@ -377,64 +393,70 @@ __device__ __forceinline__ void wave_select_stream(int n, int topk, KeyF key, Em
   const int lane = lane_id();
   const int per = (n + kWave - 1) / kWave;
   uint32_t lmax = 0;
+  int live = 0;
   for (int j = 0; j < per; ++j) {
     const int i = j * kWave + lane;
-    if (i < n) {
-      const uint32_t h = static_cast<uint32_t>(key(i) >> 32);
-      lmax = h > lmax ? h : lmax;
-    }
+    const uint64_t k = i < n ? key(i) : 0ull;
+    const uint32_t h = static_cast<uint32_t>(k >> 32);
+    lmax = h > lmax ? h : lmax;
+    live += popc64(ballot64(k != 0ull));
   }
-  const uint32_t theta = topk <= kLaneMaxTopk
-      ? lane_max_threshold(lmax, topk, reinterpret_cast<uint32_t*>(sv))
-      : wave_radix_threshold(
-            per, topk,
-            [&](int j, bool& ok) {
-              const int i = j * kWave + lane;
-              const uint64_t k = i < n ? key(i) : 0ull;
-              ok = k != 0ull;
-              return static_cast<uint32_t>(k >> 32);
-            },
-            reinterpret_cast<uint32_t*>(sv));
-  int ns = 0;
-  for (int j = 0; j < per; ++j) {
-    const int i = j * kWave + lane;
-    const uint64_t k = (i < n) ? key(i) : 0ull;
-    const bool surv = k != 0ull && static_cast<uint32_t>(k >> 32) >= theta;
-    const uint64_t m = ballot64(surv);
-    const int pos = ns + lanes_below(m);
-    if (surv && pos < kSurvCap) sv[pos] = k;
-    ns += popc64(m);
+  const auto radix = [&](uint32_t want, auto word) {
+    return wave_radix_threshold(
+        per, static_cast<int>(want),
+        [&](int j, bool& ok) {
+          const int i = j * kWave + lane;
+          return word(i < n ? key(i) : 0ull, ok);
+        },
+        reinterpret_cast<uint32_t*>(sv));
+  };
+  const auto hi_word = [](uint64_t k, bool& ok) {
+    ok = k != 0ull;
+    return static_cast<uint32_t>(k >> 32);
+  };
+  // survivors: keys of at least theta, in sv as far as it holds them
+  const auto compact = [&](uint64_t theta) {
+    int ns = 0;
+    for (int j = 0; j < per; ++j) {
+      const int i = j * kWave + lane;
+      const uint64_t k = (i < n) ? key(i) : 0ull;
+      const bool surv = k != 0ull && k >= theta;
+      const uint64_t m = ballot64(surv);
+      const int pos = ns + lanes_below(m);
+      if (surv && pos < kSurvCap) sv[pos] = k;
+      ns += popc64(m);
+    }
+    return ns;
+  };
+  uint32_t hi = 0u;
+  if (topk <= kLaneMaxTopkStream)
+    hi = lane_max_threshold(lmax, topk, reinterpret_cast<uint32_t*>(sv));
+  else if (topk > kWave || live > kSurvCap)
+    hi = radix(topk, hi_word);
+  int ns = compact(static_cast<uint64_t>(hi) << 32);
+  if (ns > kSurvCap) {
+    // score ties, or a threshold of few lanes: the exact topk-th score, and of its ties (told apart
+    // by the low word) as many as the scores above it leave room for
+    hi = radix(topk, hi_word);
+    uint32_t above = 0u;
+    for (int j = 0; j < per; ++j) {
+      const int i = j * kWave + lane;
+      above += popc64(ballot64(i < n && static_cast<uint32_t>(key(i) >> 32) > hi));
+    }
+    const uint32_t lo = radix(topk - above, [&](uint64_t k, bool& ok) {
+      ok = k != 0ull && static_cast<uint32_t>(k >> 32) == hi;
+      return static_cast<uint32_t>(k);
+    });
+    ns = compact(static_cast<uint64_t>(hi) << 32 | lo);
   }
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  if (ns <= kSurvCap) {
-    for (int i = lane; i < ns; i += kWave) {
-      const uint64_t k = sv[i];
-      int rank = 0;
-      for (int j = 0; j < ns; ++j) rank += (sv[j] > k) ? 1 : 0;
-      if (rank < topk) emit(rank, k);
-    }
-  } else {
-    uint64_t prev = ~0ull;
-    int r = 0;
-    for (; r < topk; ++r) {
-      uint64_t best = 0;
-      for (int j = 0; j < per; ++j) {
-        const int i = j * kWave + lane;
-        const uint64_t k = (i < n) ? key(i) : 0ull;
-        if (k < prev && k > best) best = k;
-      }
-#pragma unroll
-      for (int mm = 1; mm < kWave; mm <<= 1) {
-        const uint64_t o = shfl_xor_u64(best, mm);
-        best = o > best ? o : best;
-      }
-      if (best == 0ull) break;
-      if (lane == 0) emit(r, best);
-      prev = best;
-    }
-    ns = r;
+  for (int i = lane; i < ns; i += kWave) {
+    const uint64_t k = sv[i];
+    int rank = 0;
+    for (int j = 0; j < ns; ++j) rank += (sv[j] > k) ? 1 : 0;
+    if (rank < topk) emit(rank, k);
   }
   for (int p = lane; p < topk; p += kWave)
     if (p >= ns) pad(p);

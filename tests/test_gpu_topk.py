@@ -115,6 +115,36 @@ def test_topk_from_scores_threshold_edges_bitexact(topk, NC, ties):
     np.testing.assert_array_equal(got, O.topk_select(s, topk, O.Mask(**mk)))
 
 
+@pytest.mark.parametrize("topk", [30, 57, 60, 61, 64, 65, 128])
+@pytest.mark.parametrize("NC,data", [(64, "random"), (65, "ties"), (96, "random"), (97, "random"),
+                                     (5000, "random"), (5000, "ties"), (5000, "constant"),
+                                     (5000, "steps"), (5000, "hidden"), (3000, "one score")])
+def test_topk_from_scores_merge_thresholds_bitexact(topk, NC, data):
+    """Rows of one or two keys a lane, and merges of many short spans: keys above the maxima's
+    threshold that do and do not fit the survivor buffer, scores that tie in all, many or a few
+    columns (told apart by column over spans), and rows that see few columns."""
+    from omnimem_amd.index_topk import topk_from_scores
+    rng = np.random.default_rng(topk + NC)
+    MG, H = 20, 2
+    s = _scores_case(topk + NC, 1, MG, H, NC, ties=data == "ties")
+    if data == "constant":
+        s[:] = 0.25
+        s[0, ::2] = -0.0
+    elif data == "steps":  # 40 scores above 300 ties, above the rest
+        s[:] = -np.abs(np.nan_to_num(s, neginf=-9.0)) - 1.0
+        for r in s.reshape(-1, NC):
+            c = rng.permutation(NC)
+            r[c[:40]] = 1.0 + rng.standard_normal(40).astype(np.float32) ** 2
+            r[c[40:340]] = 0.5
+    elif data == "one score":
+        s[:] = -np.inf
+        s[..., NC // 2] = 3.0
+    hidden = data == "hidden"
+    got = topk_from_scores(torch.from_numpy(s).to(DEV), topk, 1, 4, 300, hidden, group_size=1)
+    mask = O.Mask(block_size=1, group_size=1, chunk_q=4, chunk_k=300, causal=int(hidden))
+    np.testing.assert_array_equal(got.cpu().numpy(), O.topk_select(s, topk, mask))
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("topk", [96, 128])
 def test_parallel_nsa_topk_fused_large_topk_bitexact(dtype, topk):
