@@ -1669,7 +1669,7 @@ __global__ __launch_bounds__(kM2Threads, 2) void topk_mfma_kernel(M2Args a) {
 // most D 2^-24 sum |q_d k_d| <= D 2^-24 |q| |k|, so with E = 4 D 2^-24 |q| max |k| |scale| (twice the
 // two bounds; it also covers the rounding of the product with scale) every column of the exact top
 // topk has s' >= x - 2 E for any x that at least topk columns reach.  x comes from bisecting the
-// row's range of s' until it leaves topk to topk + 40 columns; the candidates (about as many:
+// row's range of s' until it leaves topk to topk + kExSlack columns; the candidates (about as many:
 // random scores leave a tenth of a column within 2 E) are scored by the fmaf chain, one lane each,
 // and ranked.  A row whose norms are not between 1e-15 and 1e15 (the bound needs products and sums
 // clear of overflow and of the denormal range), whose ties leave more than kExCand candidates or
@@ -1678,12 +1678,14 @@ __global__ __launch_bounds__(kM2Threads, 2) void topk_mfma_kernel(M2Args a) {
 // gathers) at one workgroup per CU, so one row per wave and 16 waves.  Against topk_kernel, whose
 // fp32 vector scoring and selection of every column take most of its time, with the pooling: top-64
 // of 1365 columns, 16380 rows: 295 -> 137 us (top-20: 241 -> 111); top-32 of 512 columns, 6144 rows:
-// 59 -> 48 us; top-64 of 5920 columns in spans, 888 rows: 118 -> 79 us.
+// 59 -> 48 us; top-64 of 5920 columns in spans, 888 rows: 118 -> 79 us.  (ex_pays has the sizes where
+// it is no gain.)
 constexpr int kExWaves = 16;
 constexpr int kExThreads = kExWaves * kWave;
 constexpr int kExSpanCap = 1792;  // columns per item: 28 a lane, 115 KiB of scores
 constexpr int kExCand = 128;      // candidates per row, two a lane
 constexpr int kExMaxTopk = 64;
+constexpr int kExSlack = 40;      // the bisection leaves topk to topk + kExSlack columns
 constexpr float kExNorm2Min = 1e-30f, kExNorm2Max = 1e30f;
 // E is 3e-5 |q| max |k| |scale| at D = 128: the scores stay far below overflow, and E far above what
 // denormal products could lose (128 of 1.2e-38)
@@ -1876,8 +1878,8 @@ __global__ __launch_bounds__(kExThreads) void topk_exact_kernel(M2Args a) {
         }
       }
     }
-    float thr = kNegInf;  // every visible column, unless they are more than the candidate slots
-    if (nvis > kExCand) {
+    float thr = kNegInf;  // every visible column, unless a bisection would end before it starts
+    if (nvis > topk + kExSlack) {
       vmax = wave_max_xor(vmax, 1, 32);
       float lo = -wave_max_xor(-vmin, 1, 32), hi = vmax;  // at least topk columns reach lo
       bool found = false;
@@ -1893,7 +1895,7 @@ __global__ __launch_bounds__(kExThreads) void topk_exact_kernel(M2Args a) {
         }
         if (c >= topk) lo = mid;
         else hi = mid;
-        found = c >= topk && c <= topk + 40;
+        found = c >= topk && c <= topk + kExSlack;
       }
       ok = found;
       thr = lo - 2.0f * E;
@@ -2144,6 +2146,18 @@ bool ex_ok(int32_t dtype, const omm_view4& q, const omm_view4& k, int topk) {
   return topk > 16 && topk <= kExMaxTopk && (D == 64 || D == 128) && m2_view_ok(q) && m2_view_ok(k);
 }
 
+// Whether the pre-selection is the faster one of a call of few columns that topk_kernel runs in one
+// launch, pooling and all.  12 heads, top-32, topk_kernel and pre-selection: 312 rows (240 row tiles)
+// of 128 columns 20.5 and 23 us, of 200 26 and 23; 683 rows (516) of 128 35 and 43, of 200 45 and 42;
+// top-64 of 64 columns 32 and 41, of 128 50 and 52, of 160 59 and 53.  Between one row tile and two
+// per CU the tiles of a CU wait for each other's column gathers while topk_kernel is still bound by
+// its launch: 4 heads, 1365 rows (344), top-32 of 256 columns 26 and 33, of 384 34 and 36.
+bool ex_pays(int64_t B, int64_t MG, int64_t H, int64_t NC, int topk, int D, int es) {
+  if (!fused_ok(B, MG, H, NC, D, es)) return true;
+  const int64_t tiles = B * H * cdiv64(MG, kM2Rows);
+  return NC >= (topk > 32 ? 96 : 160) * (tiles > 256 && tiles <= 512 ? 2 : 1);
+}
+
 struct M2Plan {
   int span, nspan, rtiles;
   size_t ws_part;
@@ -2331,7 +2345,7 @@ extern "C" int omm_topk(const omm_view4* q, const omm_view4* k, int32_t dtype, i
   }
   // (the pre-selection's spans need other scratch than the general path's: where the given one does
   // not hold them, the general path, of the same indices, runs as it did)
-  if (ex_ok(dtype, *q, *k, topk)) {
+  if (ex_ok(dtype, *q, *k, topk) && ex_pays(B, MG, H, NC, topk, static_cast<int>(D), es)) {
     const M2Plan p = ex_plan(B, MG, H, NC, topk);
     if (p.ws_part == 0 || (workspace != nullptr && p.ws_part <= workspace_bytes)) {
       const M2Args a = m2_args(*q, *k, MG, H, NC, topk, scale, *mask, out, workspace, nullptr);
@@ -2463,7 +2477,8 @@ int topk_fused_impl(const omm_view4* q, const omm_view4* k, int32_t dtype, int32
     return launch_large(sc, B, MG, H, NC, topk, *mask, out, s);
   }
 
-  if (ex_ok(dtype, *q, *k, topk)) {  // pool once into the workspace
+  // pool once into the workspace
+  if (ex_ok(dtype, *q, *k, topk) && ex_pays(B, MG, H, NC, topk, static_cast<int>(D), es)) {
     const size_t pooled_bytes = align256(static_cast<size_t>(B * MG * H * D) * es);
     const M2Plan p = ex_plan(B, MG, H, NC, topk);
     // (a smaller or unaligned workspace, or a grid larger than the pooling's: the general path)

@@ -461,6 +461,24 @@ def test_topk_exact_preselection_matches_general_path(dtype, data, T, NC, H, D, 
             got.cpu().numpy(), O.topk(O.pool_mean(_img(q), G, name), _img(k), topk, D ** -0.5, mask))
 
 
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("NC,topk", [(95, 64), (96, 64), (105, 64), (159, 17), (160, 17), (191, 40),
+                                     (192, 40), (319, 32), (320, 32)])
+@pytest.mark.parametrize("H,rows", [(12, 312), (4, 1365), (12, 683)])
+def test_topk_exact_preselection_size_edges(NC, topk, causal, H, rows):
+    """Either side of the column counts where the pre-selection takes a call from the general kernel,
+    with up to one row tile per CU (240), up to two (344) and more (516), and of the count that its
+    bisection needs (topk + 41): both against the general path."""
+    from omnimem_amd.index_topk import parallel_nsa_topk
+    g = torch.Generator().manual_seed(NC + rows)
+    q = _bf16((1, rows, H, 64), g).to(DEV)
+    k = _bf16((1, NC, H, 64), g).to(DEV)
+    odd = torch.zeros((1, NC, H, 65), dtype=k.dtype, device=DEV)[..., :64]
+    odd.copy_(k)
+    kw = dict(block_size=2, chunk_size=57, causal=causal, group_size=1)
+    assert torch.equal(parallel_nsa_topk(q, k, topk, **kw), parallel_nsa_topk(q, odd, topk, **kw))
+
+
 @pytest.mark.parametrize("scale", [0.0, -0.5, 1e-30, 1e30, float("inf"), float("nan")])
 def test_topk_exact_preselection_scales(scale):
     """Scales whose scores overflow or leave the normal range, and the ones without an order."""
