@@ -1671,9 +1671,10 @@ __global__ __launch_bounds__(kM2Threads, 2) void topk_mfma_kernel(M2Args a) {
 // topk has s' >= x - 2 E for any x that at least topk columns reach.  x comes from bisecting the
 // row's range of s' until it leaves topk to topk + kExSlack columns; the candidates (about as many:
 // random scores leave a tenth of a column within 2 E) are scored by the fmaf chain, one lane each,
-// and ranked.  A row whose norms are not between 1e-15 and 1e15 (the bound needs products and sums
-// clear of overflow and of the denormal range), whose ties leave more than kExCand candidates or
-// whose bisection does not end scores every visible column by the chain instead.
+// and ranked.  Where ties leave more than kExCand candidates the general selection ranks them, and
+// where the norms are not between 1e-15 and 1e15 (the bound needs products and sums clear of
+// overflow and of the denormal range) it ranks every visible column; the scores of zero rows and
+// columns, padding for instance, are known without the chain.
 // Bound by the latencies of the phases between the barriers (column loads, bisection, candidate
 // gathers) at one workgroup per CU, so one row per wave and 16 waves.  Against topk_kernel, whose
 // fp32 vector scoring and selection of every column take most of its time, with the pooling: top-64
@@ -1712,6 +1713,7 @@ __global__ __launch_bounds__(kExThreads) void topk_exact_kernel(M2Args a) {
   __shared__ float qn2[kM2Rows];
   __shared__ uint32_t kn2;  // bits of the largest |k|^2 (non-negative floats order as integers)
   __shared__ int kbad;      // some |k|^2 is not finite
+  __shared__ uint32_t zcol[kExSpanCap / 16];  // columns of zeros, one bit each, 16 a word
   const int tid = threadIdx.x, lane = lane_id();
   const int w = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int l16 = lane & 15, j4 = lane >> 4;
@@ -1743,6 +1745,7 @@ __global__ __launch_bounds__(kExThreads) void topk_exact_kernel(M2Args a) {
     kn2 = 0u;
     kbad = 0;
   }
+  if (tid < kExSpanCap / 16) zcol[tid] = 0u;
   if (tid < kM2Rows * CH) {
     const int pr = tid / CH, pu = tid - pr * CH;
     uint4 val = make_uint4(0, 0, 0, 0);
@@ -1787,6 +1790,17 @@ __global__ __launch_bounds__(kExThreads) void topk_exact_kernel(M2Args a) {
       for (int i = 0; i < 4; ++i) {
         bad = bad || !(kk[i] <= kExNorm2Max);
         kmax = fmaxf(kmax, kk[i]);
+      }
+      // a column of zeros has only zero products
+      if (ballot64(kk[0] == 0.0f || kk[1] == 0.0f || kk[2] == 0.0f || kk[3] == 0.0f) != 0ull) {
+        uint32_t bits = 0u;
+#pragma unroll
+        for (int s = 0; s < SD; ++s) bits |= kf[s].x | kf[s].y | kf[s].z | kf[s].w;
+        bits &= 0x7fff7fffu;
+        bits |= static_cast<uint32_t>(__shfl_xor(static_cast<int>(bits), 16, kWave));
+        bits |= static_cast<uint32_t>(__shfl_xor(static_cast<int>(bits), 32, kWave));
+        const uint64_t z = ballot64(bits == 0u);
+        if (lane == 0) zcol[cb] = static_cast<uint32_t>(z) & 0xffffu;
       }
       *reinterpret_cast<float4*>(sc + l16 * SP + cb * 16 + 4 * j4) =
           make_float4(acc[0] * a.scale, acc[1] * a.scale, acc[2] * a.scale, acc[3] * a.scale);
@@ -1855,10 +1869,12 @@ __global__ __launch_bounds__(kExThreads) void topk_exact_kernel(M2Args a) {
   const int nvis = (rc.hi0 - rc.lo0) + (rc.hi1 - rc.lo1);
   const float q2 = qn2[r], k2 = __builtin_bit_cast(float, kn2);
   const float E = 4.0f * D * 0x1p-24f * __builtin_sqrtf(q2) * __builtin_sqrtf(k2) * fabsf(a.scale);
-  bool ok = kbad == 0 && q2 >= kExNorm2Min && q2 <= kExNorm2Max && k2 >= kExNorm2Min &&
-            E >= kExBoundMin && E <= kExBoundMax;
+  const bool bound = kbad == 0 && q2 >= kExNorm2Min && q2 <= kExNorm2Max && k2 >= kExNorm2Min &&
+                     E >= kExBoundMin && E <= kExBoundMax;
+  bool ok = bound;
   uint16_t* const list = reinterpret_cast<uint16_t*>(sv + kExCand);  // behind the candidates' keys
   int nc = 0;
+  float thr = kNegInf;  // every visible column, unless a bisection would end before it starts
   if (ok && nvis > 0) {
     // (steps past the tile's last column are skipped four at a time: a causal tile has fewer)
     float v[JM];
@@ -1878,7 +1894,6 @@ __global__ __launch_bounds__(kExThreads) void topk_exact_kernel(M2Args a) {
         }
       }
     }
-    float thr = kNegInf;  // every visible column, unless a bisection would end before it starts
     if (nvis > topk + kExSlack) {
       vmax = wave_max_xor(vmax, 1, 32);
       float lo = -wave_max_xor(-vmin, 1, 32), hi = vmax;  // at least topk columns reach lo
@@ -1898,7 +1913,7 @@ __global__ __launch_bounds__(kExThreads) void topk_exact_kernel(M2Args a) {
         found = c >= topk && c <= topk + kExSlack;
       }
       ok = found;
-      thr = lo - 2.0f * E;
+      thr = lo - 2.0f * E;  // (a bound also where the bisection did not end)
     }
     if (ok) {
 #pragma unroll
@@ -1918,9 +1933,29 @@ __global__ __launch_bounds__(kExThreads) void topk_exact_kernel(M2Args a) {
       ok = nc <= kExCand;
     }
   }
-  if (!ok) {  // wave-uniform: every visible column by the chain, then the general selection
+  if (!ok) {
+    // wave-uniform: too many candidates, or no bound.  The candidates or every visible column by the
+    // chain, then the general selection.  Zero rows and columns need no chain: with finite operands
+    // (kbad, q2) it adds zeros to its +0.
+    // (Marked in one loop and scored in another: as one loop they take 98 VGPRs and not 75, which
+    // delays the CU's next workgroup; 8196 rows of 512 columns 67 and 61 us.)
+    constexpr float kByChain = 0x1p127f;
+    const bool zeros = kbad == 0 && q2 <= kExNorm2Max;
+    bool qzero = zeros;
+    for (int d = 0; d < D; d += kWave)
+      qzero = qzero && ballot64(qf[r * D + d + lane] != 0.0f) == 0ull;
+    int nz = 0;  // zero scores so far: past topk of them none is among the best
+    for (int i0 = 0; i0 < n; i0 += kWave) {
+      const int i = i0 + lane;
+      const bool cand = i < n && in_cols(rc, i) && (!bound || srow[i] >= thr);
+      const bool z = cand && (qzero || (zeros && (zcol[i >> 4] >> (i & 15) & 1u) != 0u));
+      const uint64_t zm = ballot64(z);
+      if (cand) srow[i] = !z ? kByChain : nz + lanes_below(zm) < topk ? 0.0f * a.scale : kNegInf;
+      else if (i < n) srow[i] = kNegInf;  // hidden, or below topk others
+      nz += popc64(zm);
+    }
     for (int i = lane; i < n; i += kWave)
-      if (in_cols(rc, i)) chain(std::integral_constant<int, 1>{}, &i, &srow[i]);
+      if (srow[i] == kByChain) chain(std::integral_constant<int, 1>{}, &i, &srow[i]);
     wave_lds_fence();
     wave_select(n, topk,
                 [&](int i) -> uint64_t { return in_cols(rc, i) ? make_key(srow[i], c_begin + i, NC) : 0ull; },

@@ -409,27 +409,16 @@ def test_topk_fused_massive_ties_bitexact():
     assert (got[:, :, :2] == np.arange(16)).all()  # all-zero scores: the lowest ids
 
 
-# The exact selection of 17..64 of 16-bit rows: spans of 8, 16 and 28 column steps, one span and
-# several (the merge), rows with fewer visible columns than topk, than the candidate slots and more,
-# and the rows that leave the pre-selection: ties, infinities and NaN, norms out of its range.
-@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("data", ["random", "ties", "nonfinite", "tiny", "skewed"])
-@pytest.mark.parametrize("T,NC,H,D,G,topk,kw", [
-    (1000, 40, 2, 64, 15, 17, dict(block_size=15, chunk_size=300, causal=True)),
-    (700, 129, 3, 128, 1, 64, dict(block_size=6, chunk_size=60, causal=True)),
-    (2048, 512, 1, 128, 64, 33, dict(block_size=4, chunk_size=512, causal=True, tf_mask=True)),
-    (16380, 1365, 4, 128, 24, 64, dict(block_size=12, chunk_size=2340, causal=True)),
-    (4680, 1024, 12, 64, 9, 32, dict(block_size=64, chunk_size=4680, causal=False,
-                                     exclude_window_chunks=2, q_chunk_offset=9,
-                                     blocks_per_chunk=74, progressive_exclude=True)),
-    (2100, 1793, 24, 64, 4, 64, dict(block_size=2, chunk_size=700, causal=True)),
-    (300, 5920, 2, 128, 30, 50, dict(block_size=64, chunk_size=4680, causal=False,
-                                     exclude_window_chunks=3, q_chunk_offset=79,
-                                     blocks_per_chunk=74)),
-])
-def test_topk_exact_preselection_matches_general_path(dtype, data, T, NC, H, D, G, topk, kw):
-    from omnimem_amd.index_topk import parallel_nsa_topk
-    g = torch.Generator().manual_seed(NC + topk)
+# The exact selection of 17..64 of 16-bit rows: one span of columns (of at most 8 steps of 64, at head
+# dim 64 also 16; the wider ones are the test after this one's) and several (the merge), rows with
+# fewer visible columns than topk, than the candidate slots and more, and the rows that leave the
+# pre-selection: ties, infinities and NaN, norms out of its range, padding.
+EX_DATA = ["random", "ties", "nonfinite", "tiny", "skewed", "padded", "clusters"]
+
+
+def _ex_inputs(data, dtype, T, NC, H, D, G, seed):
+    """q, k and k with rows off 16 bytes, which takes the general path."""
+    g = torch.Generator().manual_seed(seed)
     q = torch.randn((1, T, H, D), generator=g)
     k = torch.randn((1, NC, H, D), generator=g)
     if data == "ties":
@@ -448,9 +437,39 @@ def test_topk_exact_preselection_matches_general_path(dtype, data, T, NC, H, D, 
     elif data == "skewed":  # a few columns far above the rest, the rest within rounding errors
         k = k[:, :1] + k * 2.0 ** -9
         k[:, ::97] *= 30.0
+    elif data == "padded":  # columns and rows of zeros, of either sign
+        k[:, NC // 3:, 0] = 0.0
+        k[:, 5::3, 0] = -0.0
+        k[:, NC // 5:, H - 1] = -0.0
+        q[:, T // 2:] = 0.0
+        q[:, -G:] = -0.0
+        k[:, :, H // 2] *= k[:, :, H // 2].gt(1.5).any(-1, keepdim=True)
+    elif data == "clusters":  # ties of more columns than the candidate slots hold
+        k = k[:, :6].repeat(1, NC // 6 + 1, 1, 1)[:, :NC].contiguous()
     q, k = q.to(dtype).to(DEV), k.to(dtype).to(DEV)
     odd = torch.zeros((1, NC, H, D + 1), dtype=dtype, device=DEV)[..., :D]
-    odd.copy_(k)  # rows off 16 bytes: the general path
+    odd.copy_(k)
+    return q, k, odd
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("data", EX_DATA)
+@pytest.mark.parametrize("T,NC,H,D,G,topk,kw", [
+    (1000, 40, 2, 64, 15, 17, dict(block_size=15, chunk_size=300, causal=True)),
+    (700, 129, 3, 128, 1, 64, dict(block_size=6, chunk_size=60, causal=True)),
+    (2048, 512, 1, 128, 64, 33, dict(block_size=4, chunk_size=512, causal=True, tf_mask=True)),
+    (16380, 1365, 4, 128, 24, 64, dict(block_size=12, chunk_size=2340, causal=True)),
+    (4680, 1024, 12, 64, 9, 32, dict(block_size=64, chunk_size=4680, causal=False,
+                                     exclude_window_chunks=2, q_chunk_offset=9,
+                                     blocks_per_chunk=74, progressive_exclude=True)),
+    (2100, 1793, 24, 64, 4, 64, dict(block_size=2, chunk_size=700, causal=True)),
+    (300, 5920, 2, 128, 30, 50, dict(block_size=64, chunk_size=4680, causal=False,
+                                     exclude_window_chunks=3, q_chunk_offset=79,
+                                     blocks_per_chunk=74)),
+])
+def test_topk_exact_preselection_matches_general_path(dtype, data, T, NC, H, D, G, topk, kw):
+    from omnimem_amd.index_topk import parallel_nsa_topk
+    q, k, odd = _ex_inputs(data, dtype, T, NC, H, D, G, NC + topk)
     got = parallel_nsa_topk(q, k, topk, group_size=G, **kw)
     want = parallel_nsa_topk(q, odd, topk, group_size=G, **kw)
     assert torch.equal(got, want), int((got != want).sum())
@@ -459,6 +478,39 @@ def test_topk_exact_preselection_matches_general_path(dtype, data, T, NC, H, D, 
         mask = O.Mask(block_size=15, group_size=G, chunk_q=300, chunk_k=300, causal=1)
         np.testing.assert_array_equal(
             got.cpu().numpy(), O.topk(O.pool_mean(_img(q), G, name), _img(k), topk, D ** -0.5, mask))
+
+
+@pytest.mark.parametrize("data", EX_DATA)
+@pytest.mark.parametrize("D,NC,topk,dtype,steps", [
+    (128, 500, 33, torch.bfloat16, 8), (64, 512, 64, torch.float16, 8),
+    (128, 800, 64, torch.bfloat16, 16), (64, 1024, 17, torch.bfloat16, 16),
+    (128, 1025, 64, torch.float16, 28), (64, 1025, 50, torch.bfloat16, 28),
+    (128, 1365, 64, torch.bfloat16, 28), (128, 1792, 20, torch.bfloat16, 28),
+    (64, 1792, 64, torch.float16, 28),
+])
+def test_topk_exact_preselection_one_span(D, NC, topk, dtype, steps, data):
+    """Every span size of the pre-selection in one span a row: 12 heads of 683 rows are 516 row tiles,
+    and from 512 on the columns are split only past 1792.  Past 1024 columns the rows that leave the
+    pre-selection take the streaming selection.  All heads against the general path, finite data of
+    the first and last against the oracle."""
+    from omnimem_amd.index_topk import parallel_nsa_topk
+    H, rows = 12, 683
+    assert H * -(-rows // 16) >= 512
+    assert {8: 0, 16: 512, 28: 1024}[steps] < NC <= 64 * steps
+    q, k, odd = _ex_inputs(data, dtype, rows, NC, H, D, 1, NC + topk)
+    bs = 2 if data in ("ties", "clusters") else 1
+    causal = steps < 28
+    kw = dict(block_size=bs, chunk_size=100, causal=causal, group_size=1)
+    got = parallel_nsa_topk(q, k, topk, **kw)
+    want = parallel_nsa_topk(q, odd, topk, **kw)
+    assert torch.equal(got, want), int((got != want).sum())
+    if data != "nonfinite":
+        mask = O.Mask(block_size=bs, group_size=1, chunk_q=100, chunk_k=100, causal=int(causal))
+        for h in (0, H - 1):
+            s = slice(h, h + 1)
+            np.testing.assert_array_equal(
+                got[:, :, s].cpu().numpy(),
+                O.topk(_img(q[:, :, s]), _img(k[:, :, s]), topk, D ** -0.5, mask))
 
 
 @pytest.mark.parametrize("causal", [False, True])
