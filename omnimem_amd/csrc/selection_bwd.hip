@@ -1418,11 +1418,13 @@ __global__ __launch_bounds__(NW * kWave, 2) void sel_bwd_dkv_f32_kernel(
       const float Lr[4] = {L4.x, L4.y, L4.z, L4.w}, Dr[4] = {D4.x, D4.y, D4.z, D4.w};
       const bool kv = 16 * w + l16 < cur.nv;
       float pv[4], ds[4];
-      // rows past the item's queries have zero Q / dO and lse = delta = 0, so they add nothing
+      // (rows past the item's queries have zero Q, dO, lse and delta, of which an infinite key makes
+      // NaN: they are left out by number)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        pv[r] = kv ? exp_nat(__builtin_fmaf(s4[r], scale, Lr[r])) : 0.0f;
-        ds[r] = pv[r] * (p4[r] - Dr[r]);
+        const bool in = kv && 4 * j4 + r < cur.nq;
+        pv[r] = in ? exp_nat(__builtin_fmaf(s4[r], scale, Lr[r])) : 0.0f;
+        ds[r] = in ? pv[r] * (p4[r] - Dr[r]) : 0.0f;
       }
       // dV += P^T dO and dK += dS^T Q, k-step r: queries 4 j4 + r
 #pragma unroll

@@ -149,6 +149,30 @@ def test_sel_bwd_f32_block_and_group_edges(BS, G, D):
         _close(name, got, w, *TOL[torch.float32])
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("G", [15, 16])
+def test_sel_bwd_f32_infinite_key(D, G):
+    """A key whose scores are all -inf gets zero dK and dV, also where a 16-row tile has rows without
+    a query (a ragged last group, groups of 15)."""
+    M, N, H, BS, T, chunk = 60, 210, 2, 32, 3, 45
+    gen = torch.Generator().manual_seed(G + D)
+    q, k, v = (torch.randn((1, L, H, D), generator=gen) for L in (M, N, N))
+    q[..., 0] = q[..., 0].abs() + 0.1
+    k[:, 7, :, 0] = -float("inf")
+    ids = torch.tensor([0, 1, 2], dtype=torch.int32).expand(1, -(-M // G), H, T).contiguous()
+    out, lse, do, dq, dk, dv, scale = _run(q, k, v, ids, G, BS, True, chunk, torch.float32)
+    with np.errstate(invalid="ignore"):
+        want = O.selection_attention_bwd(q.double().numpy(), k.double().numpy(), v.double().numpy(),
+                                         ids.numpy(), out.double().cpu().numpy(),
+                                         lse.double().cpu().numpy(), do.double().numpy(), G, scale,
+                                         O.dense_block_tokens(N, BS, chunk, True), chunk_size=chunk,
+                                         causal=True)
+    assert torch.count_nonzero(dk[:, 7]) == 0 and torch.count_nonzero(dv[:, 7]) == 0
+    _close("dk", dk, want[1], *TOL[torch.float32])
+    _close("dv", dv, want[2], *TOL[torch.float32])
+    _close("dq", dq[..., 1:], want[0][..., 1:], *TOL[torch.float32])
+
+
 @pytest.mark.parametrize("BS", [2, 4])
 @pytest.mark.parametrize("M,T", [(2040, 4), (2048, 4), (2100, 4), (700, 13)])
 @pytest.mark.parametrize("causal", [False, True])
