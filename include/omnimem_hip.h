@@ -3,9 +3,10 @@
  *
  * Every entry point takes plain device pointers, element strides and sizes, runs on the HIP
  * stream it is given (passed as void*, a hipStream_t), never synchronises (but for
- * omm_ids_check_end, which waits for one check), and returns an OMM_* status.  On failure omm_last_error() returns a thread-local message.  No entry point
- * allocates device memory: scratch is passed in by the caller (see the *_workspace_bytes
- * queries), so a caller's caching allocator owns every byte.
+ * omm_ids_check_end, which waits for one check), and returns an OMM_* status.  On failure
+ * omm_last_error() returns a thread-local message.  No entry point allocates device memory:
+ * scratch is passed in by the caller (see the *_workspace_bytes queries), so a caller's caching
+ * allocator owns every byte.
  *
  * Reference interfaces replaced (wuyushuwys/OmniMem, src/omnimem/nsa/...):
  *   omm_block_pool          <- K mean-pool `roped_key.view(b, s//BS, BS, n, d).mean(2)`
@@ -299,8 +300,8 @@ int omm_sel_fwd_gated(const omm_view4* q, const omm_view4* k, const omm_view4* v
  * written (0 for tokens no query sees).  Duplicated ids in a row count twice, as in the
  * forward.  Head dim 64 or 128, unit dim strides and 16-byte aligned rows run on MFMA: bf16 / f16
  * with 16-bit P and dS operands, f32 in full fp32; every other head dim <= 256 or stride runs
- * fp32 vector arithmetic.  The workspace (256-byte aligned) holds delta, -lse log2 e, the per-block CSR
- * offsets and the bucket lists. */
+ * fp32 vector arithmetic.  The workspace (256-byte aligned) holds delta, -lse (in the log the
+ * call's kernels use), the per-block CSR offsets and the bucket lists. */
 size_t omm_sel_bwd_workspace_bytes(int64_t B, int64_t M, int64_t H, int64_t N,
                                    int32_t block_size, int32_t group_size, int64_t T);
 int omm_sel_bwd(const omm_view4* q, const omm_view4* k, const omm_view4* v,

@@ -693,7 +693,8 @@ __global__ __launch_bounds__(kIdxThreads) void sel_bwd_index_kernel(
 // transposed: 16 KiB per 16 queries and 16 keys, 128 cycles of the CU's LDS against 256 of one
 // SIMD's MFMA), so rows without a query and columns without a key cost as much as real ones.  Hence
 // SUB: a tile of 16 NW query rows holds 16 NW / SUB bucket items of up to SUB queries (SUB = 16 for
-// query groups of at most 16, else 32), from as many groups.  And NW = 2 for blocks of at most 32
+// query groups of at most 16, 32 for those of at most 32 and for 2 waves, else 64), from as many
+// groups.  And NW = 2 for blocks of at most 32
 // keys, which would leave two of four waves without one.
 
 // One dword per lane: lane L's float at byte off of base (off < 0: 0) into LDS dst + 4 L, issued
@@ -1669,7 +1670,9 @@ inline size_t align256(size_t x) { return (x + 255) & ~static_cast<size_t>(255);
 struct BwdWs {
   size_t delta, nl2, offsets, groups, total;
 };
-// [delta (dense entry only) | -lse log2 e | CSR offsets | bucket lists (when dK / dV are computed)]
+// [delta (dense entry only) | -lse | CSR offsets | bucket lists (when dK / dV are computed)].  The
+// dQ kernel of a call writes -lse and its dK / dV kernel reads it: times log2 e by the 16-bit MFMA
+// kernels, natural by the fp32 MFMA kernels (the VALU kernels read the lse itself).
 inline BwdWs bwd_ws(int64_t B, int64_t M, int64_t H, int64_t MG, int64_t T, int64_t NS,
                     bool with_delta = true, bool with_index = true) {
   BwdWs w;
@@ -1729,8 +1732,8 @@ struct BwdArgs {
   float scale;
 };
 
-// Launches: dQ (and delta, -lse log2 e), the block -> group index, dK / dV.  MFMA kernels when
-// D is 64 or 128 with 16-bit rows (DM = D), else the VALU kernels with DQ dims per lane.
+// Launches: dQ (and delta, -lse), the block -> group index, dK / dV.  MFMA kernels when D is 64 or
+// 128 with rows of 16-byte alignment (DM = D), else the VALU kernels with DQ dims per lane.
 template <typename QT, int DM, int DQ>
 int sel_bwd_launch(const BwdArgs& a, char* ws, const BwdWs& L, hipStream_t s) {
   const omm_view4 &q = *a.q, &k = *a.k, &v = *a.v, &ids = *a.ids;
@@ -1875,13 +1878,8 @@ int sel_bwd_ptr_launch(const PtrBwdArgs& a, char* ws, const BwdWs& L, hipStream_
 template <typename QT>
 int sel_bwd_typed(const BwdArgs& a, bool mfma, char* ws, const BwdWs& L, hipStream_t s) {
   const int64_t D = a.q->size[3];
-  if constexpr (sizeof(QT) == 2) {
-    if (mfma && D == 128) return sel_bwd_launch<QT, 128, 0>(a, ws, L, s);
-    if (mfma && D == 64) return sel_bwd_launch<QT, 64, 0>(a, ws, L, s);
-  } else {
-    if (mfma && D == 128) return sel_bwd_launch<QT, 128, 0>(a, ws, L, s);
-    if (mfma && D == 64) return sel_bwd_launch<QT, 64, 0>(a, ws, L, s);
-  }
+  if (mfma && D == 128) return sel_bwd_launch<QT, 128, 0>(a, ws, L, s);
+  if (mfma && D == 64) return sel_bwd_launch<QT, 64, 0>(a, ws, L, s);
   if (D <= 64) return sel_bwd_launch<QT, 0, 16>(a, ws, L, s);
   if (D <= 128) return sel_bwd_launch<QT, 0, 32>(a, ws, L, s);
   return sel_bwd_launch<QT, 0, 64>(a, ws, L, s);

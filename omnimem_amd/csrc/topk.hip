@@ -1665,10 +1665,11 @@ __global__ __launch_bounds__(kM2Threads, 2) void topk_mfma_kernel(M2Args a) {
 
 // ---- MFMA pre-selection with exact scores (16 < topk <= 64) --------------------------------------
 // The same inputs as above, but the indices are those of the fmaf-chain scores (topk_kernel's), bit
-// for bit.  MFMA scores s' pick the candidates: both sums differ from the exact dot product by at
-// most D 2^-24 sum |q_d k_d| <= D 2^-24 |q| |k|, so with E = 4 D 2^-24 |q| max |k| |scale| (twice the
-// two bounds; it also covers the rounding of the product with scale) every column of the exact top
-// topk has s' >= x - 2 E for any x that at least topk columns reach.  x comes from bisecting the
+// for bit.  MFMA scores s' pick the candidates.  The chain, which rounds to nearest, differs from the
+// exact dot product by at most D 2^-24 sum |q_d k_d| <= D 2^-24 |q| |k|, and the matrix unit's sum of
+// exact products, whose rounding inside is not stated (by truncation at every addition at worst), by
+// twice that.  So with E = 4 D 2^-24 |q| max |k| |scale| (the rest covers the product with scale)
+// every column of the exact top topk has s' >= x - 2 E for any x that at least topk columns reach.  x comes from bisecting the
 // row's range of s' until it leaves topk to topk + kExSlack columns; the candidates (about as many:
 // random scores leave a tenth of a column within 2 E) are scored by the fmaf chain, one lane each,
 // and ranked.  Where ties leave more than kExCand candidates the general selection ranks them, and
