@@ -5,8 +5,8 @@ finite differences and by torch autograd) is fed the same bf16/f16 inputs and th
 own (out, lse), so the comparison isolates the backward kernels.  Tolerance, per gradient tensor
 g with oracle value r: max|g - r| <= 2e-2 * max|r| and mean|g - r| <= 5e-3 * mean|r| (16-bit
 MFMA operands for P and dS, fp32 accumulation, one rounding of the result to the input dtype);
-fp32 inputs (full fp32 VALU arithmetic, BASELINE's fp32 bar): 1e-4 * max|r| and 1e-5 * mean|r|.
-Head dims other than 64 / 128, fp32 and non-unit dim strides run the VALU kernels.
+fp32 inputs (full fp32 arithmetic, BASELINE's fp32 bar): 1e-4 * max|r| and 1e-5 * mean|r|.
+Head dims other than 64 / 128, rows off 16 bytes and non-unit dim strides run the VALU kernels.
 
 Cases follow the forward's (reference rules: cuda_backend/csrc/selection_bwd.cu:18-306,
 inverted_index.cu:13-34, bwd_common.cuh:33-60): partial tail blocks, chunk-causal prefixes, -1
@@ -50,11 +50,14 @@ def _close(name, got, want, mx=2e-2, mean=5e-3):
         f"{name}: mean-abs {err.mean():.3e} > {mean} x {scale_mean:.3e}")
 
 
-def _run(q, k, v, ids, G, BS, causal, chunk, dtype, scale=None, seed=0):
+def _run(q, k, v, ids, G, BS, causal, chunk, dtype, scale=None, seed=0, off16=False):
     from omnimem_amd.selection import sel_fwd, sel_bwd
     D = q.shape[-1]
     scale = D ** -0.5 if scale is None else scale
     qd, kd, vd, idd = (x.to(DEV) for x in (q, k, v, ids))
+    if off16:  # rows of k off 16 bytes
+        kd = torch.nn.functional.pad(kd, (0, 1))[..., :D]
+        assert kd.stride(2) == D + 1
     out, lse = sel_fwd(qd, kd, vd, idd, BS, chunk, scale, causal, G)
     gen = torch.Generator().manual_seed(seed + 1)
     do = torch.randn(q.shape, generator=gen).to(dtype)
@@ -79,6 +82,8 @@ CASES_VALU = [
     # M, N, H, D, G, BS, T, causal, chunk, minus, dup
     (256, 512, 2, 128, 64, 64, 4, False, 1, 0.0, False),
     (300, 700, 3, 128, 15, 30, 8, True, 600, 0.1, False),
+    (130, 256, 2, 64, 64, 32, 5, False, 1, 0.2, True),
+    (100, 180, 2, 40, 15, 30, 4, True, 60, 0.1, False),
     (200, 333, 2, 96, 100, 100, 3, True, 150, 0.0, True),
     (90, 180, 1, 200, 30, 16, 6, True, 60, 0.2, False),
 ]
@@ -193,21 +198,18 @@ def test_sel_bwd_index_pair_lists(BS, M, T, causal):
         _close(name, got, w)
 
 
-# fp32 everywhere; bf16 only at head dims the MFMA kernels do not take (bf16 at 64 / 128 runs
-# the MFMA kernels, covered by test_sel_bwd_matches_oracle)
 VALU_PARAMS = [pytest.param(case, dt, id=f"valu{i}-{'f32' if dt == torch.float32 else 'bf16'}")
-               for i, case in enumerate(CASES_VALU) for dt in (torch.float32, torch.bfloat16)
-               if not (dt == torch.bfloat16 and case[3] in (64, 128))]
+               for i, case in enumerate(CASES_VALU) for dt in (torch.float32, torch.bfloat16)]
 
 
 @pytest.mark.parametrize("case,dtype", VALU_PARAMS)
 def test_sel_bwd_valu_matches_oracle(case, dtype):
-    """fp32 everywhere, and bf16 at head dims the MFMA kernels do not take (96, 200)."""
+    """Head dims that the MFMA kernels do not take (40, 96, 200), and 64 and 128 in rows off 16 bytes."""
     M, N, H, D, G, BS, T, causal, chunk, minus, dup = case
     gen = torch.Generator().manual_seed(hash(case) % 997)
     q, k, v = (torch.randn((1, L, H, D), generator=gen).to(dtype) for L in (M, N, N))
     ids = _ids(gen, 1, -(-M // G), H, T, -(-N // BS), minus, dup)
-    out, lse, do, dq, dk, dv, scale = _run(q, k, v, ids, G, BS, causal, chunk, dtype)
+    out, lse, do, dq, dk, dv, scale = _run(q, k, v, ids, G, BS, causal, chunk, dtype, off16=True)
     want = O.selection_attention_bwd(q.double().numpy(), k.double().numpy(), v.double().numpy(),
                                      ids.numpy(), out.double().cpu().numpy(),
                                      lse.double().cpu().numpy(), do.double().numpy(), G, scale,
