@@ -689,13 +689,14 @@ __global__ __launch_bounds__(kIdxThreads) void sel_bwd_index_kernel(
 // LDS and memory waits are covered by the other's work.  The item's lse arrives already as
 // -lse log2 e (written by the dQ kernel), and the softmax scale of dK is applied once to the sums.
 //
-// The kernel is bound by its LDS reads (every wave reads each Q / dO row twice, as rows and
-// transposed: 16 KiB per 16 queries and 16 keys, 128 cycles of the CU's LDS against 256 of one
-// SIMD's MFMA), so rows without a query and columns without a key cost as much as real ones.  Hence
-// SUB: a tile of 16 NW query rows holds 16 NW / SUB bucket items of up to SUB queries (SUB = 16 for
-// query groups of at most 16, 32 for those of at most 32 and for 2 waves, else 64), from as many
-// groups.  And NW = 2 for blocks of at most 32
-// keys, which would leave two of four waves without one.
+// LDS is the kernel's busiest unit: every wave reads each Q / dO row twice, as rows and transposed, 16
+// KiB per 16 queries and 16 keys (46% of the CU's cycles at blocks and groups of 64, the MFMA 38%; a
+// third of the wave cycles wait for copies and barriers).  So rows without a query and columns
+// without a key cost as much as real ones.  Hence SUB: a tile of 16 NW query rows holds 16 NW / SUB
+// bucket items of up to SUB queries (SUB = 16 for query groups of at most 16, 32 for those of at most
+// 32 and for 2 waves, else 64), from as many groups.  And NW = 2 for blocks of at most 32 keys, which
+// would leave two of four waves without one; there the waits weigh most (41% of the wave cycles at
+// blocks of 30 and groups of 15, LDS 32%, MFMA 25%).
 
 // One dword per lane: lane L's float at byte off of base (off < 0: 0) into LDS dst + 4 L, issued
 // like dma_part (inline asm, ordered by the kernel's own waits).
