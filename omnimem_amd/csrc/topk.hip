@@ -2380,10 +2380,12 @@ extern "C" int omm_topk(const omm_view4* q, const omm_view4* k, int32_t dtype, i
     return launch_m2<false>(dtype, static_cast<int>(D), a, B, H, p, s);
   }
   // (the pre-selection's spans need other scratch than the general path's: where the given one does
-  // not hold them, the general path, of the same indices, runs as it did)
+  // not hold both, the general path, of the same indices, runs or refuses as it did)
   if (ex_ok(dtype, *q, *k, topk) && ex_pays(B, MG, H, NC, topk, static_cast<int>(D), es)) {
     const M2Plan p = ex_plan(B, MG, H, NC, topk);
-    if (p.ws_part == 0 || (workspace != nullptr && p.ws_part <= workspace_bytes)) {
+    const size_t need = std::max(
+        p.ws_part, make_plan(B, MG, H, NC, topk, static_cast<int>(D), es, false, false).ws_part);
+    if (need == 0 || (workspace != nullptr && need <= workspace_bytes)) {
       const M2Args a = m2_args(*q, *k, MG, H, NC, topk, scale, *mask, out, workspace, nullptr);
       return launch_ex(dtype, static_cast<int>(D), a, B, H, p, s);
     }
@@ -2517,8 +2519,14 @@ int topk_fused_impl(const omm_view4* q, const omm_view4* k, int32_t dtype, int32
   if (ex_ok(dtype, *q, *k, topk) && ex_pays(B, MG, H, NC, topk, static_cast<int>(D), es)) {
     const size_t pooled_bytes = align256(static_cast<size_t>(B * MG * H * D) * es);
     const M2Plan p = ex_plan(B, MG, H, NC, topk);
-    // (a smaller or unaligned workspace, or a grid larger than the pooling's: the general path)
-    if (workspace != nullptr && pooled_bytes + p.ws_part <= workspace_bytes &&
+    const size_t part =
+        fused_ok(B, MG, H, NC, static_cast<int>(D), es)
+            ? p.ws_part
+            : std::max(p.ws_part, make_plan(B, MG, H, NC, topk, static_cast<int>(D), es, false,
+                                            false).ws_part);
+    // (a workspace that is unaligned or holds less than this path's and the general one's need, or a
+    // grid larger than the pooling's: the general path, which runs or refuses as it did)
+    if (workspace != nullptr && pooled_bytes + part <= workspace_bytes &&
         (reinterpret_cast<uintptr_t>(workspace) & 15u) == 0 && MG <= 65535 && B <= 65535) {
       omm_view4 pooled{};
       pooled.data = workspace;

@@ -531,6 +531,28 @@ def test_topk_exact_preselection_size_edges(NC, topk, causal, H, rows):
     assert torch.equal(parallel_nsa_topk(q, k, topk, **kw), parallel_nsa_topk(q, odd, topk, **kw))
 
 
+@pytest.mark.parametrize("aligned", [True, False])
+def test_topk_exact_preselection_refuses_small_workspaces(aligned):
+    """A workspace too small for the general path's column spans (24 of 128 for 12 rows of 3000
+    columns, 73,728 bytes) is refused also where the pre-selection's 6 spans would fit it."""
+    from omnimem_amd import _lib
+    from omnimem_amd.backend import NSABackendError
+    from omnimem_amd.index_topk import _mask
+    q = torch.zeros((1, 12, 1, 128), dtype=torch.bfloat16, device=DEV)
+    k = torch.zeros((1, 3000, 1, 128 if aligned else 129), dtype=torch.bfloat16, device=DEV)[..., :128]
+    out = torch.empty((1, 12, 1, 32), dtype=torch.int32, device=DEV)
+    m = _mask(1, 1, 12, 12, False, 0, 0, False, False, 0, 0, 0, 0)
+    assert _lib.lib().omm_topk_workspace_bytes(1, 12, 1, 3000, 32) >= 73728
+    ws = torch.empty((128 * 1024,), dtype=torch.uint8, device=DEV)
+    for name, args, pooled in (("omm_topk", (32,), 0), ("omm_topk_fused", (1, 32), 12 * 256)):
+        def call(n):
+            _lib.call(name, _lib.view4(q), _lib.view4(k), _lib.dtype_code(q), *args, 1.0, m,
+                      out.data_ptr(), ws.data_ptr(), n, _lib.stream_of(q))
+        call(pooled + 73728)
+        with pytest.raises(NSABackendError, match="workspace"):
+            call(pooled + 73727)
+
+
 @pytest.mark.parametrize("scale", [0.0, -0.5, 1e-30, 1e30, float("inf"), float("nan")])
 def test_topk_exact_preselection_scales(scale):
     """Scales whose scores overflow or leave the normal range, and the ones without an order."""
